@@ -48,10 +48,11 @@
 //
 // Rows whose keys all carry one mask bias m, small enough products given
 // (constant_mask_row), have the same weights fl-softmax(m + bias) on every
-// such row: attention_const_kernel runs only O^T for them, four rows per
-// work item.  For the block, const_weights_kernel first forms those weights
-// once for the m of the first such row, and lists the four-row chunks of
-// that m and of any other m; the constant-mask launches walk those lists.
+// such row.  For the block, pair_bias_kernel forms those weights once for
+// the m of the first such row, and the fast launch applies them to each such
+// row's V (shared_row_item).  attention_const_kernel serves the others (the
+// staged layout's, and rows of another m): four rows per work item share one
+// softmax.
 #include "attn_common.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
@@ -97,38 +98,50 @@ __device__ __forceinline__ int v_position(int g) {
 // Rows whose mask bias is one finite nonzero value m on every key < n
 // (padding rows: inf (mask - 1) = -1e9), when the products are bounded below
 // half the float32 spacing next to m on either side: then fl(s + m) = m for
-// every key (|s| <= 32 max|q| max|k|, with a margin for the native rounding
-// of s), so the native logit fl(fl(s + m) + bias) is fl(m + bias), the same
+// every key (|s| <= max|q|_2 max|k|_2 over the row's queries and keys, with a
+// margin for the native rounding of s), so the native logit fl(fl(s + m) + bias) is fl(m + bias), the same
 // for every such row.  With |m| = f 2^e, f in [0.5, 1), the spacing above
 // |m| is 2^(e - 24); toward zero it is the same unless |m| is a power of two
-// (f = 0.5), where it halves.
+// (f = 0.5), where it halves.  The row's own 2-norms bound s about 7 times
+// closer than 32 max|q| max|k| over the whole pair would (unit-scale q and k
+// at N = 1536: 16 against 114, the limit at m = -1e9 being 32), which keeps
+// ordinary padding rows off the exact softmax: 184 rows of 1536 take 0.3 ms
+// with their shared weights against 1.10 ms there.
 __device__ __forceinline__ bool constant_mask_row(const AttnArgs& a, int b, float& m) {
   if (a.magnitudes == nullptr || a.magnitudes[4] != 1u) return false;
+  if (!constant_mask(a.tile_flags, b, m)) return false;
   const uint32_t* f3 =
       a.tile_flags + ((int64_t)b * kTileFlagParts + kTileFlagMaxPart) * kTileFlagWords;
-  const float hi = __builtin_bit_cast(float, f3[0]);
-  const float lo = __builtin_bit_cast(float, f3[1]);
-  // false for NaN anywhere, for an infinite m and for m = 0
-  if (!(hi == lo && __builtin_fabsf(hi) < INFINITY && hi != 0.f)) return false;
-  const float mq = __builtin_bit_cast(float, a.magnitudes[0]);
-  const float mk = __builtin_bit_cast(float, a.magnitudes[1]);
-  const float s_bound = 32.0f * mq * mk * (1.0f + 0x1p-10f);
-  const bool power_of_two = (__builtin_bit_cast(uint32_t, hi) & 0x7fffffu) == 0u;
+  // 2^-120 covers squares that underflow (32 of them, each below 2^-126)
+  const float q2 = __builtin_bit_cast(float, f3[kRowNormQ]) + 0x1p-120f;
+  const float k2 = __builtin_bit_cast(float, f3[kRowNormK]) + 0x1p-120f;
+  const float s_bound = __builtin_sqrtf(q2) * __builtin_sqrtf(k2) * (1.0f + 0x1p-10f);
+  const bool power_of_two = (__builtin_bit_cast(uint32_t, m) & 0x7fffffu) == 0u;
   const float half_ulp =
-      __builtin_ldexpf(1.0f, __builtin_amdgcn_frexp_expf(hi) - (power_of_two ? 26 : 25));
-  m = hi;
-  return s_bound < half_ulp;
+      __builtin_ldexpf(1.0f, __builtin_amdgcn_frexp_expf(m) - (power_of_two ? 26 : 25));
+  return s_bound < half_ulp;  // false for a NaN bound
+}
+
+// The block's constant-mask rows of the m that const_m[0] holds: their
+// weights are formed once for the whole call (pair_bias_kernel), and the fast
+// launch serves them (shared_row_item).
+__device__ __forceinline__ bool shared_weight_row(const AttnArgs& a, int b) {
+  float m;
+  return a.const_m != nullptr && constant_mask_row(a, b, m) &&
+         a.const_m[0] == __builtin_bit_cast(uint32_t, m);
 }
 
 // The constant-row kernel serves chunks of kConstRows consecutive outer
 // rows: the rows of a chunk that satisfy constant_mask_row with the m of
-// the chunk's first such row.  The exact launch leaves exactly those out.
+// the chunk's first row of a constant mask bias (whatever that row's bound,
+// so that the m of a chunk is known before the norms are).  The exact launch
+// leaves exactly those out.
 __device__ __forceinline__ bool const_chunk_member(const AttnArgs& a, int b) {
   float m;
   if (!constant_mask_row(a, b, m)) return false;
   for (int r = b - b % kConstRows; r < b; ++r) {
     float mr;
-    if (constant_mask_row(a, r, mr)) return mr == m;
+    if (constant_mask(a.tile_flags, r, mr)) return mr == m;
   }
   return true;  // the chunk's first constant-mask row
 }
@@ -198,12 +211,139 @@ __device__ __forceinline__ bool row_is_fast(const AttnArgs& a, int b, int nkt_al
   return fast;
 }
 
-// Rows served by the exact launch: neither fast nor taken by the
-// constant-row kernel.
+// Rows served by the exact launch: neither fast, nor served with shared
+// weights, nor taken by the constant-row kernel.
 __device__ __forceinline__ bool row_is_exact(const AttnArgs& a, int b, int nkt_all) {
   int nkt;
   uint32_t mw[kTileFlagWords], any;
-  return !row_is_fast(a, b, nkt_all, nkt, mw, any) && !const_chunk_member(a, b);
+  return !row_is_fast(a, b, nkt_all, nkt, mw, any) && !shared_weight_row(a, b) &&
+         !const_chunk_member(a, b);
+}
+
+// One work item (b, h, qt) of the rows with shared weights (kAttnBlock): the
+// weights' fp16 planes P' = P 2^kVShift of the (head, 32-query tile) are
+// loaded as the other rows load a bias fragment, and only O^T += V^T P'^T
+// runs: no K tiles, no S^T, no softmax, 6 MFMAs per row and key tile.  One
+// v^T exponent per head, so the products accumulate into O directly and the
+// factor 2^-(e_v + kVShift) is applied in the epilogue.
+//
+// The fast launch runs these items where their rows fall in its grid: its
+// work-groups for these rows would otherwise leave at once.  A work-group
+// takes rows b and b + 1 when both are such rows (b even), so each weight
+// fragment, 4 KB per wave and tile from L2 and the bound of this loop, is
+// loaded once for two rows; a row alone runs twice over.  A ring stage holds
+// a tile's V^T planes of both rows (wave w copies plane w % 2 of row w / 2).
+// 184 such rows at N = 1536 add 0.3 ms to the fast launch (0.5 with a row
+// per work-group); their own launch (four rows per work-group, 250 VGPRs)
+// took 0.36 ms, and 17 us for 25 rows at N = 256, all latency, where this
+// adds 1 us.
+__device__ __forceinline__ void shared_row_item(const AttnArgs& a, int nkt, int b, int h, int qt,
+                                                uint8_t* ring) {
+  if ((b & 1) && shared_weight_row(a, b - 1)) return;  // served with row b - 1
+  const bool two = !(b & 1) && b + 1 < a.batch && shared_weight_row(a, b + 1);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5;
+  const int l32 = lane & 31;
+  const int jq = qt * kBq + 32 * w + l32;
+  const int64_t nt = a.np >> 5;
+  const int64_t slice_bytes = (int64_t)a.np * 128;
+  const int last = nkt - 1;
+  const __amdgpu_buffer_rsrc_t rp =
+      buffer(reinterpret_cast<const float*>(a.const_p + (((int64_t)h * nt + qt * 4 + w) * nkt) * 4096),
+             (int64_t)nkt * 4096);
+  const uint32_t ob = (uint32_t)lane * 16;
+
+  const int64_t bh = (int64_t)(b + (two ? w >> 1 : 0)) * kHeads + h;
+  const uint8_t* dma_base = reinterpret_cast<const uint8_t*>(a.v) + bh * slice_bytes +
+                            (w & 1) * (slice_bytes >> 1);
+  const uint32_t dma_voff = (uint32_t)((lane >> 2) * 64 + 16 * ((lane & 3) ^ swz(lane >> 2)));
+  const uint32_t dma_lds = lds_address(ring) + (uint32_t)w * kPlaneBytes;
+  auto copy = [&](int t) {
+    const uint8_t* src = dma_base + (int64_t)min(t, last) * kPlaneBytes;
+    const uint32_t dst = dma_lds + (uint32_t)(t & 3) * kStageBytes;
+    lds_dma16_s(dma_voff, src, dst);
+    lds_dma16_s(dma_voff + 1024, src, dst + 1024);
+  };
+  auto load = [&](int t) -> f32x16 {  // ph[0], ph[1], pl[0], pl[1]
+    const uint32_t so = (uint32_t)min(t, last) * 4096;
+    return cat4(buffer_f4(rp, ob, so), buffer_f4(rp, ob + 1024, so), buffer_f4(rp, ob + 2048, so),
+                buffer_f4(rp, ob + 3072, so));
+  };
+  const uint32_t rd0 = l32 * 64 + 16 * (half ^ swz(l32));
+  const uint32_t rd1 = l32 * 64 + 16 * ((2 + half) ^ swz(l32));
+
+  f32x16 o0 = {}, o1 = {};
+  auto products = [&](const f32x16& x, int t) {
+    const uint8_t* base = ring + (t & 3) * kStageBytes;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const uint8_t* at = base + (m ? rd1 : rd0);
+      const bf16x8 vh0 = *(const bf16x8*)(at), vl0 = *(const bf16x8*)(at + kPlaneBytes);
+      const bf16x8 vh1 = *(const bf16x8*)(at + 2 * kPlaneBytes);
+      const bf16x8 vl1 = *(const bf16x8*)(at + 3 * kPlaneBytes);
+      const bf16x8 ph = __builtin_bit_cast(
+          bf16x8, f32x4{x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]});
+      const bf16x8 pl = __builtin_bit_cast(
+          bf16x8, f32x4{x[8 + 4 * m], x[9 + 4 * m], x[10 + 4 * m], x[11 + 4 * m]});
+      o0 = mfma_f16(vl0, ph, o0);
+      o1 = mfma_f16(vl1, ph, o1);
+      o0 = mfma_f16(vh0, pl, o0);
+      o1 = mfma_f16(vh1, pl, o1);
+      o0 = mfma_f16(vh0, ph, o0);
+      o1 = mfma_f16(vh1, ph, o1);
+    }
+  };
+  // Tile t sits in stage t % 4.  Iteration t starts tile t + 3 into the
+  // stage that held tile t - 1, which every wave left behind at the previous
+  // barrier.  Tiles past the last are clamped (in range, never used).
+  f32x16 x_a = load(0);
+  copy(0);
+  f32x16 x_b = load(1);
+  copy(1);
+  copy(2);
+  wait_vmcnt<0>();
+  __syncthreads();
+  auto body = [&](f32x16& x, int t) {
+    products(x, t);
+    if (t == last) return;
+    x = load(t + 2);
+    copy(t + 3);
+    // Tile t + 1 has landed once at most this iteration's four weight loads
+    // and two copies, and the previous iteration's two copies (tile t + 2,
+    // issued after its weight loads), are outstanding.  When tile t + 2 is
+    // past the last, the compiler may drop its weight loads: wait for all.
+    if (t + 2 <= last)
+      wait_vmcnt<8>();
+    else
+      wait_vmcnt<0>();
+    __syncthreads();
+  };
+  for (int t = 0; t <= last; t += 2) {
+    body(x_a, t);
+    if (t + 1 <= last) body(x_b, t + 1);
+  }
+  wait_vmcnt<0>();  // the clamped copies land before the LDS is released
+
+  if (jq >= a.n) return;
+  const int64_t per = (int64_t)kHeads * nt;
+  const float sc = __builtin_ldexpf(
+      a.scales[2 * (int64_t)a.batch * per + (int64_t)b * per + (int64_t)h * nt], -kVShift);
+  const float l_tot = a.const_l[h * a.np + jq];
+  auto store = [&](const f32x16& o, int row) {
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      const int64_t col = h * kHeadDim + 8 * rr + 4 * half;
+      f32x4 ov4 = {o[4 * rr + 0] * sc / l_tot, o[4 * rr + 1] * sc / l_tot,
+                   o[4 * rr + 2] * sc / l_tot, o[4 * rr + 3] * sc / l_tot};
+      if (a.gate)
+        ov4 = ov4 * *(const f32x4*)(a.gate + ((int64_t)row * a.np + jq) * kHidden + col);
+      *(f32x4*)(a.out + ((int64_t)row * a.n + jq) * kHidden + col) = ov4;
+    }
+  };
+  store(o0, b);
+  if (two) store(o1, b + 1);
 }
 
 // Both layouts read q, k and v^T in the plane layout (ProjArgs::planes) with
@@ -280,12 +420,17 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, int nqt, int nkt_
   int nkt;
   const bool fast = row_is_fast(a, b, nkt_all, nkt, mw, any);
   // Each row runs in the launch of its softmax path (uniform per work-group).
-  if (fast == EXACT) return;
+  if (fast == EXACT) {
+    if constexpr (kBlock && !EXACT) {
+      if (shared_weight_row(a, b)) shared_row_item(a, nkt_all, b, h, qt, lds);
+    }
+    return;
+  }
   // Exact rows that the constant-row kernel serves are left out; other
   // constant-mask rows (another m than their chunk's) still skip S^T here.
   if (EXACT && const_chunk_member(a, b)) return;
   // The block's fast launch reads the log2 bias relative to each query's
-  // reference (launch_bias_reference): x' = x - C_q + kRelOffset.
+  // reference (launch_pair_bias): x' = x - C_q + kRelOffset.
   const bool rel = kBlock && !EXACT && a.magnitudes != nullptr &&
                    a.magnitudes[kRelativeBiasWord] == 1u;
   float m_row = 0.f;
@@ -755,20 +900,30 @@ typedef float ConstScales[kTileFlagWords * 32];  // 2^-(e_t + kVShift) per tile 
 // kConstRows chunk + r) and their m; uniform across the work-group.
 __device__ __forceinline__ uint32_t const_chunk_rows(const AttnArgs& a, int chunk, float& m_row) {
   uint32_t live = 0u;
+  bool found = false;
   m_row = 0.f;
   for (int r = 0; r < kConstRows; ++r) {
     const int b = chunk * kConstRows + r;
     float m = 0.f;
-    if (b < a.batch && constant_mask_row(a, b, m) && (live == 0u || m == m_row)) {
-      if (live == 0u) m_row = m;
-      live |= 1u << r;
-    }
+    if (b >= a.batch || !constant_mask(a.tile_flags, b, m)) continue;
+    if (!found) m_row = m;
+    found = true;
+    if (m == m_row && constant_mask_row(a, b, m)) live |= 1u << r;
   }
   return live;
 }
 
+// The m of a chunk's first row of a constant mask bias, if it has one.
+__device__ __forceinline__ bool const_chunk_mask(const AttnArgs& a, int chunk, float& m) {
+  for (int r = 0; r < kConstRows; ++r) {
+    const int b = chunk * kConstRows + r;
+    if (b < a.batch && constant_mask(a.tile_flags, b, m)) return true;
+  }
+  return false;
+}
+
 // One work item: the chunk's constant-mask rows for (head, query tile) hq.
-template <int LAYOUT, bool LOADED>
+template <int LAYOUT>
 __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, int chunk, int hq,
                                            uint8_t* ring, ConstScales* Sv) {
   constexpr bool kBlock = LAYOUT == kAttnBlock;
@@ -779,15 +934,6 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   float m_row = 0.f;
   const uint32_t live = __builtin_amdgcn_readfirstlane(const_chunk_rows(a, chunk, m_row));
   if (live == 0u) return;
-  // Chunks whose m has the block's precomputed weights (const_weights_kernel,
-  // formed once per (head, 32-query tile)) belong to the LOADED launch: its
-  // tile loop loads those weights in place of the bias fragments and runs
-  // no softmax.  The other launch serves every other chunk.
-  const bool has_weights = kBlock && a.const_m != nullptr &&
-                           __builtin_amdgcn_readfirstlane(a.const_m[0]) ==
-                               __builtin_bit_cast(uint32_t, m_row);
-  if (has_weights != LOADED) return;
-  constexpr bool loaded = LOADED;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -799,14 +945,7 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   const int qt32 = (j0 >> 5) + w;
   const int64_t nt = a.np >> 5;
   const int64_t frag = ((int64_t)h * nt + qt32) * nt * 1024;
-  // Per key tile 4 KB at the same lane offsets: the bias fragment (x), or
-  // the loaded weights' planes (ph[0], ph[1], pl[0], pl[1] in x's four
-  // 16-byte parts).
-  const __amdgpu_buffer_rsrc_t rb =
-      loaded ? buffer(reinterpret_cast<const float*>(
-                          a.const_p + (((int64_t)h * nt + qt32) * nkt) * 4096),
-                      (int64_t)nkt * 4096)
-             : buffer(a.bias + frag, nt * 4096);
+  const __amdgpu_buffer_rsrc_t rb = buffer(a.bias + frag, nt * 4096);
   const uint32_t ob = (uint32_t)lane * 16;
   const int64_t slice_bytes = (int64_t)a.np * 128;
 
@@ -853,7 +992,6 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   // Logits of tile t from its bias fragment: fl(m + bias), -inf past key n.
   const int full_tiles = a.n / kBk;
   auto finish = [&](f32x16& x, int t) {
-    if constexpr (loaded) return;
     if (t < full_tiles) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) x[r] = m_row + x[r];
@@ -877,13 +1015,6 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   // P = exp2(x log2(e) - c_ref) w_ref (at most 2^8 by the lazy max), into
   // fp16 planes as P 2^kVShift.
   auto softmax = [&](const f32x16& x, bf16x8 (&ph)[2], bf16x8 (&pl)[2]) {
-    if constexpr (loaded) {
-      ph[0] = __builtin_bit_cast(bf16x8, f32x4{x[0], x[1], x[2], x[3]});
-      ph[1] = __builtin_bit_cast(bf16x8, f32x4{x[4], x[5], x[6], x[7]});
-      pl[0] = __builtin_bit_cast(bf16x8, f32x4{x[8], x[9], x[10], x[11]});
-      pl[1] = __builtin_bit_cast(bf16x8, f32x4{x[12], x[13], x[14], x[15]});
-      return;
-    }
     const float mt = xor32_max(max16(x));
     if (__any(mt > m_ref + kRescaleNat)) {
       const float m_new = __builtin_elementwise_maximum(m_ref, mt);
@@ -918,41 +1049,6 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   // same for every row, so there the products accumulate into O_r directly
   // and the factor is applied once in the epilogue.
   auto pv = [&](int stage, int t, const bf16x8 (&ph)[2], const bf16x8 (&pl)[2]) {
-    if constexpr (kBlock && loaded) {
-      // Every row's operands are read first and the 24 products issued row
-      // by row within each term, so consecutive MFMAs are independent and no
-      // LDS read waits on the MFMA before it.  Rows that are not live run on
-      // whatever their stage holds (their copies are skipped) and are never
-      // stored.
-      bf16x8 vh[kConstRows][2], vl[kConstRows][2];
-      for_const_rows([&](auto rc) {
-        constexpr int r = decltype(rc)::value;
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-          vh[r][m] = plane_rd(stage, r, 0, m);
-          vl[r][m] = plane_rd(stage, r, 1, m);
-        }
-      });
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        for_const_rows([&](auto rc) {
-          constexpr int r = decltype(rc)::value;
-          f32x16& orow = const_row<r>(o);
-          orow = mfma_f16(vl[r][m], ph[m], orow);
-        });
-        for_const_rows([&](auto rc) {
-          constexpr int r = decltype(rc)::value;
-          f32x16& orow = const_row<r>(o);
-          orow = mfma_f16(vh[r][m], pl[m], orow);
-        });
-        for_const_rows([&](auto rc) {
-          constexpr int r = decltype(rc)::value;
-          f32x16& orow = const_row<r>(o);
-          orow = mfma_f16(vh[r][m], ph[m], orow);
-        });
-      }
-      return;
-    }
     for_const_rows([&](auto rc) {
       constexpr int r = decltype(rc)::value;
       if (!((live >> r) & 1u)) return;
@@ -1033,7 +1129,7 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   }
   wait_vmcnt<0>();  // the clamped tail loads land before the LDS is released
 
-  const float l_tot = loaded ? a.const_l[h * a.np + jq] : xor32_sum(l_run);
+  const float l_tot = xor32_sum(l_run);
   if (jq < a.n) {
     for_const_rows([&](auto rc) {
       constexpr int r = decltype(rc)::value;
@@ -1059,55 +1155,232 @@ __device__ __forceinline__ void const_item(const AttnArgs& a, int nqt, int nkt, 
   }
 }
 
-// The weights of the block's constant-mask rows, once for every such row
-// (const_item's loaded path).  Every row whose keys all carry the mask bias
-// m of the first constant-mask row has the logits x = fl(m + bias) for each
-// (head, query, key), whatever its outer row.  One work-group per (head,
-// 32-query tile), wave w on key tiles w, w + 4, ...: pass 1 each query's max
-// m_q over all keys; pass 2 the exact softmax's weights with the reference
-// at that max, P = exp2(x log2(e) - c) w, c = fl(m_q log2(e)),
-// w = 2^-(m_q log2(e) - c) (equal quantised logits get equal weights), their
-// sum l_q, and P 2^kVShift split into fp16 planes in the P.V operand order,
-// stored as the four 16-byte parts of a bias fragment.  With no
-// constant-mask row, const_m[0] becomes a NaN (no row's m matches it).
-// Work-group 0 also writes the two chunk lists of the constant-mask launches
-// (AttnArgs::const_m): the chunks whose rows have that m, and the others.
-__global__ __launch_bounds__(kThreads) void const_weights_kernel(AttnArgs a, int nkt) {
+// A work-group per item: the few items with work spread over the whole
+// chip as the empty ones leave (a grid that walks the items would give some
+// work-groups one item more than others).  The loop serves any grid.
+template <int LAYOUT>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+void attention_const_kernel(AttnArgs a, int nqt, int nkt, int nchunks, uint32_t items) {
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kConstStages * kStageBytesC];
+  __shared__ ConstScales Sv[kConstRows];
+  // XCD x serves the (head, query tile) pairs [x H nqt / 8, (x + 1) H nqt / 8)
+  // of every chunk, chunk-major.
+  const int nhq = kHeads * nqt;
+  const int xcd = (int)(blockIdx.x % kXcds);
+  const int hq0 = xcd * nhq / kXcds;
+  const int nh = (xcd + 1) * nhq / kXcds - hq0;
+  if (nh == 0) return;
+  if (LAYOUT == kAttnBlock && a.const_m != nullptr) {
+    // The block's chunk list (pair_bias_kernel): a persistent grid, a
+    // multiple of kXcds work-groups, walks it.
+    const int count = (int)__builtin_amdgcn_readfirstlane(a.const_m[2]);
+    const uint32_t* list = a.const_m + kConstListWord;
+    const int stride = (int)(gridDim.x / kXcds);
+    for (int slot = (int)(blockIdx.x / kXcds); slot < nh * count; slot += stride) {
+      const int chunk = (int)__builtin_amdgcn_readfirstlane(list[slot / nh]);
+      const_item<LAYOUT>(a, nqt, nkt, chunk, hq0 + slot % nh, ring, Sv);
+      __syncthreads();
+    }
+    return;
+  }
+  // Every (chunk, pair) item, one work-group each (the items without
+  // constant-mask rows leave at once).
+  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+    const int slot = (int)(item / kXcds);
+    if (slot < nh * nchunks) {
+      const_item<LAYOUT>(a, nqt, nkt, slot / nh, hq0 + slot % nh, ring, Sv);
+      __syncthreads();
+    }
+  }
+}
+
+// Row norms (kRowNormQ, kRowNormK) of one head of outer row b from its q and
+// k planes in the block's layout, when its mask bias is constant: the 2-norms
+// of the hi planes (|x| <= |hi| (1 + 2^-11) + 2^-25 in scaled units), four
+// lanes per 32-channel row.  Formed here, off the few rows that need them,
+// rather than in the projection's epilogue, whose tile loop compiled 10%
+// slower with them.
+template <int kT>
+__device__ __forceinline__ void row_norms(const AttnArgs& a, uint32_t* tile_flags, int b, int h,
+                                          float (*red)[32]) {
+  float m;
+  if (!constant_mask(a.tile_flags, b, m)) return;
+  const int tid = threadIdx.x;
+  const int64_t slice_bytes = (int64_t)a.np * 128;
+  const int64_t nt = a.np >> 5;
+  const int64_t bh = (int64_t)b * kHeads + h;
+#pragma unroll
+  for (int op = 0; op < 2; ++op) {
+    const uint8_t* src = reinterpret_cast<const uint8_t*>(op == 0 ? a.q : a.k) + bh * slice_bytes;
+    float top = 0.f;
+#pragma unroll 4
+    for (int c = tid; c < 4 * a.np; c += kT) {
+      const f16x8 v = __builtin_bit_cast(f16x8, *(const bf16x8*)(src + (int64_t)c * 16));
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)v[e], (float)v[e], s);
+      s += dpp<0xB1>(s);
+      s += dpp<0x4E>(s);
+      top = __builtin_elementwise_maximum(top, s);
+    }
+    top = wave_max(top);
+    if ((tid & 63) == 0) red[op][tid >> 6] = top;
+  }
+  __syncthreads();
+  if (tid < 2) {
+    float top = red[tid][0];
+    for (int i = 1; i < kT / 64; ++i) top = __builtin_elementwise_maximum(top, red[tid][i]);
+    const float inv = a.scales[((int64_t)tid * a.batch * kHeads + bh) * nt];
+    note_row_norm(tile_flags, b, tid,
+                  __builtin_fmaf(top, 1.0f + 0x1p-9f, 0x1p-34f) * inv * inv);
+  }
+}
+
+// What the block's attention needs before it starts (launch_pair_bias), one
+// work-group per (head, 32-query tile): the relative log2 bias of the fast
+// softmax, and the shared weights of the constant-mask rows.  With kWeights,
+// one more work-group per (outer row, head) for row_norms.  Lane (half, l32) of a fragment holds 16 keys of query l32
+// (bias_frag_index), so a query's largest value over a set of tiles is a
+// per-lane max, an xor-32 max and a max over the waves (wave w takes tiles
+// w, w + kBiasWaves, ...).  Bound by latency: a few tiles per wave in
+// sequence, so eight waves per work-group rather than four, and one launch
+// rather than two (8.3 us with the row norms against 4.8 + 7.7 us at
+// N = 256; 89 against 28 + 36 at N = 1536, where the norms read 145 MB).
+//
+// Relative bias.  T is the first 32-key tile with a nonzero mask bias,
+// minimised over the rows that have an unmasked key (so keys of tiles t < T
+// are unmasked on every row the fast softmax serves); nkt when no row has a
+// masked key.  C_q = ceil of query q's largest log2 bias over tiles t < T;
+// every tile of the query is then rewritten as bias_l2 - (C_q - kRelOffset),
+// one rounding.  With T = 0 nothing is rewritten and the flag stays 0.
+//
+// Shared weights (kWeights: the call has a mask; else no row has a constant
+// mask bias).  Every row whose keys all carry the mask bias m of the first
+// constant-mask row has the logits x = fl(m + bias) for each (head, query,
+// key), whatever its outer row.  Pass 1 each query's max m_q over all keys;
+// pass 2 the exact softmax's weights with the reference at that max,
+// P = exp2(x log2(e) - c) w, c = fl(m_q log2(e)), w = 2^-(m_q log2(e) - c)
+// (equal quantised logits get equal weights), their sum l_q, and P 2^kVShift
+// split into fp16 planes in the P.V operand order, stored as the four
+// 16-byte parts of a bias fragment.  With no constant-mask row, const_m[0]
+// becomes a NaN (no row's m matches it).  Work-group 0 also counts the
+// chunks whose rows have that m (const_m[1]) and lists the others.
+constexpr int kBiasWaves = 8;
+template <bool kWeights>
+__global__ __launch_bounds__(kBiasWaves * 64) void pair_bias_kernel(AttnArgs a, float* bias_l2,
+                                                                    uint32_t* magnitudes,
+                                                                    uint32_t* tile_flags) {
+  constexpr int kT = kBiasWaves * 64;
+  __shared__ int wmin[kBiasWaves];
+  __shared__ float red[kBiasWaves][32];
   __shared__ int first;
   __shared__ int counts[2];
-  __shared__ float red[kThreads / 64][32];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = tid >> 6;
   const int half = lane >> 5;
   const int l32 = lane & 31;
+  const int nkt = (a.n + kBk - 1) / kBk;
   const int nt = a.np >> 5;
   const int h = (int)blockIdx.x / nt;
   const int qt32 = (int)blockIdx.x % nt;
-  if (tid == 0) first = a.batch;
-  __syncthreads();
-  for (int b = tid; b < a.batch; b += kThreads) {
-    float m;
-    if (constant_mask_row(a, b, m)) {
-      atomicMin(&first, b);
-      break;
-    }
+  if (kWeights && h >= kHeads) {
+    const int bh = (int)blockIdx.x - kHeads * nt;
+    row_norms<kT>(a, tile_flags, bh / kHeads, bh % kHeads, red);
+    return;
   }
+  if (kWeights && tid == 0) first = a.batch;
+  if (kWeights) __syncthreads();
+  int t_first = nkt;
+  int b_first = a.batch;
+  for (int b = tid; b < a.batch; b += kT) {
+    const uint32_t* f = a.tile_flags + (int64_t)b * kTileFlagParts * kTileFlagWords;
+    uint32_t open = 0u;
+    int t0 = nkt;
+#pragma unroll
+    for (int i = 0; i < kTileFlagWords; ++i) {
+      const int lo = 32 * i;
+      const uint32_t valid =
+          nkt >= lo + 32 ? 0xffffffffu : nkt > lo ? (1u << (nkt - lo)) - 1u : 0u;
+      open |= ~f[kTileFlagWords + i] & valid;
+      const uint32_t m = f[i] & valid;
+      if (t0 == nkt && m != 0u) t0 = lo + __builtin_ctz(m);
+    }
+    if (open != 0u) t_first = min(t_first, t0);
+    float m;
+    if (kWeights && b_first == a.batch && constant_mask(a.tile_flags, b, m)) b_first = b;
+  }
+  if (kWeights && b_first < a.batch) atomicMin(&first, b_first);
+  // wave minimum, then the work-group's
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) t_first = min(t_first, __shfl_xor(t_first, d));
+  if (lane == 0) wmin[w] = t_first;
   __syncthreads();
+  int T = wmin[0];
+#pragma unroll
+  for (int i = 1; i < kBiasWaves; ++i) T = min(T, wmin[i]);
+  // The largest of every wave's value for this lane's query.
+  auto over_waves = [&](float v) -> float {
+    v = xor32_max(v);
+    __syncthreads();
+    if (half == 0) red[w][l32] = v;
+    __syncthreads();
+    float r = red[0][l32];
+#pragma unroll
+    for (int i = 1; i < kBiasWaves; ++i) r = __builtin_elementwise_maximum(r, red[i][l32]);
+    return r;
+  };
+  const int64_t frag = ((int64_t)h * nt + qt32) * nt * 1024 + lane * 4;
+  auto load16 = [&](const float* src) -> f32x16 {
+    return cat4(*(const f32x4*)src, *(const f32x4*)(src + 256), *(const f32x4*)(src + 512),
+                *(const f32x4*)(src + 768));
+  };
+
+  if (T > 0) {  // uniform
+    float m = -INFINITY;
+    for (int t = w; t < T; t += kBiasWaves)
+      m = __builtin_elementwise_maximum(m, max16(load16(bias_l2 + frag + (int64_t)t * 1024)));
+    // |C_q| < 2^22 whenever the fast softmax runs (its logit bound); other
+    // values are never read, and keep the copy as it is
+    const float c = __builtin_ceilf(over_waves(m));
+    const float shift = __builtin_fabsf(c) < 4194304.0f ? c - kRelOffset : 0.0f;
+    for (int t = w; t < nt; t += kBiasWaves) {
+      float* dst = bias_l2 + frag + (int64_t)t * 1024;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f32x4 v = *(const f32x4*)(dst + 256 * i);
+        v = v - shift;
+        *(f32x4*)(dst + 256 * i) = v;
+      }
+    }
+    if (blockIdx.x == 0 && tid == 0) magnitudes[kRelativeBiasWord] = 1u;
+  }
+  if constexpr (!kWeights) {
+    if (blockIdx.x == 0 && tid == 0) {
+      a.const_m[0] = 0x7fc00000u;
+      a.const_m[1] = 0u;
+      a.const_m[2] = 0u;
+    }
+    return;
+  }
+
   const int b0 = first;
   float m_c = 0.f;
-  const bool any = b0 < a.batch && constant_mask_row(a, b0, m_c);
+  const bool any = b0 < a.batch && constant_mask(a.tile_flags, b0, m_c);
   const uint32_t m_bits = any ? __builtin_bit_cast(uint32_t, m_c) : 0x7fc00000u;
   if (blockIdx.x == 0) {
     if (tid < 2) counts[tid] = 0;
     __syncthreads();
     const int nchunks = (a.batch + kConstRows - 1) / kConstRows;
-    for (int c = tid; c < nchunks; c += kThreads) {
-      float m_row;
-      if (const_chunk_rows(a, c, m_row) == 0u) continue;
-      const int list = __builtin_bit_cast(uint32_t, m_row) == m_bits ? 0 : 1;
-      const int at = atomicAdd(&counts[list], 1);
-      a.const_m[kConstListWord + list * nchunks + at] = (uint32_t)c;
+    if (any) {
+      for (int c = tid; c < nchunks; c += kT) {
+        float m_row;
+        if (!const_chunk_mask(a, c, m_row)) continue;
+        const bool other = __builtin_bit_cast(uint32_t, m_row) != m_bits;
+        const int at = atomicAdd(&counts[other], 1);
+        if (other) a.const_m[kConstListWord + at] = (uint32_t)c;
+      }
     }
     __syncthreads();
     if (tid == 0) {
@@ -1118,14 +1391,9 @@ __global__ __launch_bounds__(kThreads) void const_weights_kernel(AttnArgs a, int
   }
   if (!any) return;
 
-  const __amdgpu_buffer_rsrc_t rb =
-      buffer(a.bias + ((int64_t)h * nt + qt32) * nt * 1024, (int64_t)nt * 4096);
-  const uint32_t ob = (uint32_t)lane * 16;
   const int full_tiles = a.n / kBk;
   auto logits = [&](int t) -> f32x16 {
-    const uint32_t so = (uint32_t)t * 4096;
-    f32x16 x = cat4(buffer_f4(rb, ob, so), buffer_f4(rb, ob + 1024, so),
-                    buffer_f4(rb, ob + 2048, so), buffer_f4(rb, ob + 3072, so));
+    f32x16 x = load16(a.bias + frag + (int64_t)t * 1024);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int key = t * kBk + 8 * (r >> 2) + 4 * half + (r & 3);
@@ -1134,20 +1402,14 @@ __global__ __launch_bounds__(kThreads) void const_weights_kernel(AttnArgs a, int
     return x;
   };
   float mx = -INFINITY;
-  for (int t = w; t < nkt; t += kThreads / 64) mx = __builtin_elementwise_maximum(mx, max16(logits(t)));
-  mx = xor32_max(mx);
-  if (half == 0) red[w][l32] = mx;
-  __syncthreads();
-  const float m_q = __builtin_elementwise_maximum(
-      __builtin_elementwise_maximum(red[0][l32], red[1][l32]),
-      __builtin_elementwise_maximum(red[2][l32], red[3][l32]));
-  __syncthreads();
+  for (int t = w; t < nkt; t += kBiasWaves) mx = __builtin_elementwise_maximum(mx, max16(logits(t)));
+  const float m_q = over_waves(mx);
   const float c = m_q * kLog2e;
   const float wr = exp2_fast(-__builtin_fmaf(m_q, kLog2e, -c));
   const float f = wr * (float)(1 << kVShift);
-  uint8_t* const dst = a.const_p + (((int64_t)h * nt + qt32) * nkt) * 4096 + ob;
+  uint8_t* const dst = a.const_p + (((int64_t)h * nt + qt32) * nkt) * 4096 + lane * 16;
   float ps = 0.f;
-  for (int t = w; t < nkt; t += kThreads / 64) {
+  for (int t = w; t < nkt; t += kBiasWaves) {
     const f32x16 x = logits(t);
     bf16x8 ph[2], pl[2];
 #pragma unroll
@@ -1167,130 +1429,15 @@ __global__ __launch_bounds__(kThreads) void const_weights_kernel(AttnArgs a, int
     *(bf16x8*)(d + 3072) = pl[1];
   }
   ps = xor32_sum(ps);
+  __syncthreads();
   if (half == 0) red[w][l32] = ps;
   __syncthreads();
-  if (tid < 32)
-    a.const_l[h * a.np + qt32 * 32 + tid] =
-        ((red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid])) * wr;
-}
-
-// A work-group per item: the few items with work spread over the whole
-// chip as the empty ones leave (a grid that walks the items would give some
-// work-groups one item more than others).  The loop serves any grid.
-// LOADED: the chunks with precomputed weights (no softmax registers, three
-// work-groups per CU, as many as the LDS holds); the other launch keeps two.
-template <int LAYOUT, bool LOADED>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(2, 2)))
-void attention_const_kernel(AttnArgs a, int nqt, int nkt, int nchunks, uint32_t items) {
-  __shared__ __attribute__((aligned(16))) uint8_t ring[kConstStages * kStageBytesC];
-  __shared__ ConstScales Sv[kConstRows];
-  // XCD x serves the (head, query tile) pairs [x H nqt / 8, (x + 1) H nqt / 8)
-  // of every chunk, chunk-major.
-  const int nhq = kHeads * nqt;
-  const int xcd = (int)(blockIdx.x % kXcds);
-  const int hq0 = xcd * nhq / kXcds;
-  const int nh = (xcd + 1) * nhq / kXcds - hq0;
-  if (nh == 0) return;
-  if (LAYOUT == kAttnBlock && a.const_m != nullptr) {
-    // The block's chunk lists (const_weights_kernel): a persistent grid, a
-    // multiple of kXcds work-groups, walks this launch's list.
-    const int count = (int)__builtin_amdgcn_readfirstlane(a.const_m[LOADED ? 1 : 2]);
-    const uint32_t* list = a.const_m + kConstListWord + (LOADED ? 0 : nchunks);
-    const int stride = (int)(gridDim.x / kXcds);
-    for (int slot = (int)(blockIdx.x / kXcds); slot < nh * count; slot += stride) {
-      const int chunk = (int)__builtin_amdgcn_readfirstlane(list[slot / nh]);
-      const_item<LAYOUT, LOADED>(a, nqt, nkt, chunk, hq0 + slot % nh, ring, Sv);
-      __syncthreads();
-    }
-    return;
-  }
-  // Every (chunk, pair) item, one work-group each (the items without
-  // constant-mask rows leave at once).
-  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
-    const int slot = (int)(item / kXcds);
-    if (slot < nh * nchunks) {
-      const_item<LAYOUT, LOADED>(a, nqt, nkt, slot / nh, hq0 + slot % nh, ring, Sv);
-      __syncthreads();
-    }
-  }
-}
-
-// The relative log2 bias of the block (launch_bias_reference).  One
-// work-group per (head, 32-query tile); every work-group first finds T, the
-// first 32-key tile with a nonzero mask bias, minimised over the rows that
-// have an unmasked key (so keys of tiles t < T are unmasked on every row the
-// fast softmax serves); nkt when no row has a masked key.  Lane (half, l32)
-// of a fragment holds 16 keys of query l32 (bias_frag_index), so a query's
-// largest log2 bias over tiles t < T is a per-lane max, an xor-32 max and a
-// max over the four waves (each takes every fourth tile).  C_q = ceil of it;
-// every tile of the query is then rewritten as bias_l2 - (C_q - kRelOffset),
-// one rounding.  With T = 0 nothing is rewritten and the flag stays 0.
-__global__ __launch_bounds__(256) void bias_reference_kernel(const uint32_t* __restrict__ flags,
-                                                             int batch, int n, int np,
-                                                             float* __restrict__ bias_l2,
-                                                             uint32_t* __restrict__ magnitudes) {
-  __shared__ int wmin[4];
-  __shared__ float qmax[4][32];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = tid >> 6;
-  const int nkt = (n + kBk - 1) / kBk;
-  const int nt = np >> 5;
-  int t_first = nkt;
-  for (int b = tid; b < batch; b += 256) {
-    const uint32_t* f = flags + (int64_t)b * kTileFlagParts * kTileFlagWords;
-    uint32_t open = 0u;
-    int first = nkt;
+  if (tid < 32) {
+    float l = 0.f;
 #pragma unroll
-    for (int i = 0; i < kTileFlagWords; ++i) {
-      const int lo = 32 * i;
-      const uint32_t valid =
-          nkt >= lo + 32 ? 0xffffffffu : nkt > lo ? (1u << (nkt - lo)) - 1u : 0u;
-      open |= ~f[kTileFlagWords + i] & valid;
-      const uint32_t m = f[i] & valid;
-      if (first == nkt && m != 0u) first = lo + __builtin_ctz(m);
-    }
-    if (open != 0u) t_first = min(t_first, first);
+    for (int i = 0; i < kBiasWaves; ++i) l += red[i][tid];
+    a.const_l[h * a.np + qt32 * 32 + tid] = l * wr;
   }
-  // wave minimum, then the work-group's
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) t_first = min(t_first, __shfl_xor(t_first, d));
-  if (lane == 0) wmin[w] = t_first;
-  __syncthreads();
-  const int T = min(min(wmin[0], wmin[1]), min(wmin[2], wmin[3]));
-  if (T == 0) return;  // uniform
-  const int h = (int)blockIdx.x / nt;
-  const int qt = (int)blockIdx.x % nt;
-  float* frag = bias_l2 + ((int64_t)h * nt + qt) * nt * 1024 + lane * 4;
-  float m = -INFINITY;
-  for (int t = w; t < T; t += 4) {
-    const float* src = frag + (int64_t)t * 1024;
-    const f32x16 x = cat4(*(const f32x4*)src, *(const f32x4*)(src + 256),
-                          *(const f32x4*)(src + 512), *(const f32x4*)(src + 768));
-    m = __builtin_elementwise_maximum(m, max16(x));
-  }
-  m = xor32_max(m);
-  if (lane < 32) qmax[w][lane] = m;
-  __syncthreads();
-  const int q = lane & 31;
-  const float mq = __builtin_elementwise_maximum(
-      __builtin_elementwise_maximum(qmax[0][q], qmax[1][q]),
-      __builtin_elementwise_maximum(qmax[2][q], qmax[3][q]));
-  // |C_q| < 2^22 whenever the fast softmax runs (its logit bound); other
-  // values are never read, and keep the copy as it is
-  const float c = __builtin_ceilf(mq);
-  const float shift = __builtin_fabsf(c) < 4194304.0f ? c - kRelOffset : 0.0f;
-  for (int t = w; t < nt; t += 4) {
-    float* dst = frag + (int64_t)t * 1024;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f32x4 v = *(const f32x4*)(dst + 256 * i);
-      v = v - shift;
-      *(f32x4*)(dst + 256 * i) = v;
-    }
-  }
-  if (blockIdx.x == 0 && tid == 0) magnitudes[kRelativeBiasWord] = 1u;
 }
 
 }  // namespace
@@ -1307,11 +1454,11 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
     return hipErrorInvalidValue;
   const size_t mask_row_bytes = (size_t)nkt * kBk * sizeof(float);
   const int ppg = pair_group_size(nqt, (uint64_t)kBq * (uint64_t)a.np * sizeof(float));
-  // Three launches: rows on the fast softmax path (one work-group per work
-  // item; the others leave after reading their row's flags), then the other
-  // rows (fully masked rows, rows whose logits are not bounded) on a
-  // persistent grid, then the constant-mask rows (padding rows), a chunk of
-  // kConstRows at a time, one work-group per item.
+  // Three launches: rows on the fast softmax path and the block's rows with
+  // shared weights (one work-group per work item; the others leave after
+  // reading their row's flags), then the other rows (rows whose logits are
+  // not bounded) on a persistent grid, then the constant-mask rows without
+  // shared weights, a chunk of kConstRows at a time, one work-group per item.
   const uint32_t exact_grid =
       (uint32_t)std::min<uint64_t>((uint64_t)a.batch * kExactChunks, kExactGroups);
   const int nchunks = (a.batch + kConstRows - 1) / kConstRows;
@@ -1326,25 +1473,15 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
     hipLaunchKernelGGL((attention_split_kernel<kAttnBlock, true>), dim3(exact_grid),
                        dim3(kThreads), mask_row_bytes, stream, a, nqt, nkt, (uint32_t)total, ppg);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    if (a.const_m != nullptr) {
-      // the shared weights and the chunk lists, then both constant-mask
-      // launches on persistent grids (two work-groups per CU) over them
-      if (a.const_l == nullptr || a.const_p == nullptr) return hipErrorInvalidValue;
-      hipLaunchKernelGGL(const_weights_kernel, dim3((uint32_t)(kHeads * (a.np >> 5))),
-                         dim3(kThreads), 0, stream, a, nkt);
-      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-      int cap = device_cu_count() * 2;
-      cap -= cap % kXcds;
-      const uint32_t grid = (uint32_t)std::max(cap, kXcds);
-      hipLaunchKernelGGL((attention_const_kernel<kAttnBlock, true>), dim3(grid), dim3(kThreads), 0,
-                         stream, a, nqt, nkt, nchunks, (uint32_t)const_items);
-      if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-      hipLaunchKernelGGL((attention_const_kernel<kAttnBlock, false>), dim3(grid), dim3(kThreads), 0,
-                         stream, a, nqt, nkt, nchunks, (uint32_t)const_items);
-    } else {
-      hipLaunchKernelGGL((attention_const_kernel<kAttnBlock, false>), dim3(const_grid),
-                         dim3(kThreads), 0, stream, a, nqt, nkt, nchunks, (uint32_t)const_items);
-    }
+    if (!a.has_mask) return hipSuccess;  // no row has a constant mask bias
+    // constant-mask rows without shared weights, on a persistent grid (two
+    // work-groups per CU) over their chunk list
+    int cap = device_cu_count() * 2;
+    cap -= cap % kXcds;
+    const uint32_t grid =
+        a.const_m != nullptr ? (uint32_t)std::max(cap, kXcds) : (uint32_t)const_items;
+    hipLaunchKernelGGL((attention_const_kernel<kAttnBlock>), dim3(grid), dim3(kThreads), 0, stream,
+                       a, nqt, nkt, nchunks, (uint32_t)const_items);
   } else if (layout == kAttnStaged) {
     hipLaunchKernelGGL((attention_split_kernel<kAttnStaged, false>), dim3((uint32_t)total),
                        dim3(kThreads), mask_row_bytes, stream, a, nqt, nkt, (uint32_t)total, ppg);
@@ -1352,7 +1489,7 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
     hipLaunchKernelGGL((attention_split_kernel<kAttnStaged, true>), dim3(exact_grid),
                        dim3(kThreads), mask_row_bytes, stream, a, nqt, nkt, (uint32_t)total, ppg);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-    hipLaunchKernelGGL((attention_const_kernel<kAttnStaged, false>), dim3(const_grid), dim3(kThreads), 0,
+    hipLaunchKernelGGL((attention_const_kernel<kAttnStaged>), dim3(const_grid), dim3(kThreads), 0,
                        stream, a, nqt, nkt, nchunks, (uint32_t)const_items);
   } else {
     return hipErrorInvalidValue;
@@ -1360,13 +1497,20 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
   return hipGetLastError();
 }
 
-hipError_t launch_bias_reference(const uint32_t* flags, int batch, int n, int np, float* bias_l2,
-                                 uint32_t* magnitudes, hipStream_t stream) {
-  if (batch <= 0 || n <= 0) return hipSuccess;
-  if (np % kBq || np < n || round_up(n, kBk) / kBk > kTileFlagWords * 32 || magnitudes == nullptr)
+hipError_t launch_pair_bias(const AttnArgs& a, float* bias_l2, uint32_t* magnitudes,
+                            uint32_t* tile_flags, hipStream_t stream) {
+  if (a.batch <= 0 || a.n <= 0) return hipSuccess;
+  if (a.np % kBq || a.np < a.n || round_up(a.n, kBk) / kBk > kTileFlagWords * 32 ||
+      magnitudes == nullptr || a.const_m == nullptr || a.const_l == nullptr || a.const_p == nullptr)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(bias_reference_kernel, dim3((uint32_t)(kHeads * (np >> 5))), dim3(256), 0,
-                     stream, flags, batch, n, np, bias_l2, magnitudes);
+  const uint32_t tiles = (uint32_t)(kHeads * (a.np >> 5));
+  const dim3 threads(kBiasWaves * 64);
+  if (a.has_mask)
+    hipLaunchKernelGGL(pair_bias_kernel<true>, dim3(tiles + (uint32_t)a.batch * kHeads), threads, 0, stream,
+                       a, bias_l2, magnitudes, tile_flags);
+  else
+    hipLaunchKernelGGL(pair_bias_kernel<false>, dim3(tiles), threads, 0, stream, a, bias_l2,
+                       magnitudes, tile_flags);
   return hipGetLastError();
 }
 
@@ -1383,13 +1527,16 @@ hipError_t launch_bias_reference(const uint32_t* flags, int batch, int n, int np
 //         keys in v_position order) times 2^e (e = value_plane_exp of the
 //         tile's max |value|) as fp16 hi and lo planes, and 2^-e at
 //         scales[((2 batch + b) 4 + h) (np / 32) + t].
+// tile_flags (nullable): on rows of one finite nonzero mask bias, the tile's
+// largest squared row norm of q or k is added to kRowNormQ / kRowNormK.
 // partial (nullable): each work-group's NaN-propagating max |q|, |k|, |v| at
 // partial[3 blockIdx.x + op] (0 for operands it did not stage), reduced by
 // reduce_magnitudes_kernel.  Each wave transposes v through its own LDS
 // tile.
 __global__ __launch_bounds__(256) void stage_planes_kernel(AttnArgs a, uint8_t* qp, uint8_t* kp,
                                                            uint8_t* vp, float* scales,
-                                                           float* partial, int64_t waves) {
+                                                           float* partial, uint32_t* tile_flags,
+                                                           int64_t waves) {
   __shared__ float tv[4][32][33];
   __shared__ float wmax[4][3];
   const int lane = threadIdx.x & 63;
@@ -1428,6 +1575,16 @@ __global__ __launch_bounds__(256) void stage_planes_kernel(AttnArgs a, uint8_t* 
     if (op < 2) {
       if (op == 0) mq = m;
       else mk = m;
+      float m_row;
+      if (tile_flags != nullptr && constant_mask(tile_flags, b, m_row)) {
+        // row r's 32 channels sit in the lane pair (2r, 2r + 1)
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s += (x[i].x * x[i].x + x[i].y * x[i].y) + (x[i].z * x[i].z + x[i].w * x[i].w);
+        s = wave_max(s + dpp<0xB1>(s));
+        if (lane == 0) note_row_norm(tile_flags, b, op, s);
+      }
       int e = plane_exp(m);
       e = e < -kPlaneExpMax ? -kPlaneExpMax : e > kPlaneExpMax ? kPlaneExpMax : e;
       const float f = __builtin_ldexpf(1.0f, e);
@@ -1533,7 +1690,7 @@ int64_t stage_planes_groups(const AttnArgs& a) {
 
 hipError_t launch_stage_planes(const AttnArgs& a, void* q_planes, void* k_planes, void* v_planes,
                                float* scales, float* partial, uint32_t* magnitudes,
-                               hipStream_t stream) {
+                               uint32_t* tile_flags, hipStream_t stream) {
   const int64_t waves = 3 * (int64_t)a.batch * kHeads * (a.np / 32);
   if (waves == 0) return hipSuccess;
   const int64_t blocks = stage_planes_groups(a);
@@ -1541,7 +1698,7 @@ hipError_t launch_stage_planes(const AttnArgs& a, void* q_planes, void* k_planes
   if ((partial == nullptr) != (magnitudes == nullptr)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(stage_planes_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, a,
                      static_cast<uint8_t*>(q_planes), static_cast<uint8_t*>(k_planes),
-                     static_cast<uint8_t*>(v_planes), scales, partial, waves);
+                     static_cast<uint8_t*>(v_planes), scales, partial, tile_flags, waves);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || magnitudes == nullptr) return e;
   const int64_t rgroups = (blocks + 255) / 256 < 256 ? (blocks + 255) / 256 : 256;

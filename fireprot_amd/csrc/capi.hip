@@ -37,8 +37,8 @@ size_t elem_bytes(int dtype) { return dtype == FPX_BF16 ? 2 : 4; }
 //   tile flags [n][kTileFlagParts * kTileFlagWords] uint32, then the
 //   kMagnitudeWords words of the magnitude record; scales [3][n][4][np / 32]
 //   float (the plane layout's per-tile inverse scales of q, k and v^T); FP32
-//   only: the constant-mask rows' weights and chunk lists (AttnArgs::const_m,
-//   const_l, const_p: kConstListWord words and two lists of
+//   only: the constant-mask rows' weights and chunk list (AttnArgs::const_m,
+//   const_l, const_p: kConstListWord words and room for two lists of
 //   ceil(n / kConstRows) chunk indices, l [4][np] float, the planes
 //   [4][np / 32][ceil(n / 32)] x 4 KB).
 // FP32 blocks hold q, k and v^T in the fp16 plane layout (ProjArgs), in the
@@ -135,6 +135,59 @@ T* as(char* p) {
   return reinterpret_cast<T*>(p);
 }
 
+// The FP32 block's attention operands in its workspace.
+fpx::AttnArgs block_attention_args(const BlockPointers& w, int n, bool has_mask) {
+  fpx::AttnArgs a{};
+  a.q = as<float>(w.qh);
+  a.k = as<float>(w.kh);
+  a.v = as<float>(w.vt);
+  a.mbias = w.mbias;
+  a.mb_stride = w.np;
+  a.bias = as<float>(w.tri);
+  a.bias_l2 = as<float>(w.tri) + (size_t)fpx::kHeads * w.np * w.np;
+  a.bias_stride = w.np;
+  a.bias_rows = w.np;
+  a.gate = as<float>(w.gs);
+  a.out = as<float>(w.og);
+  a.tile_flags = w.flags;
+  a.magnitudes = w.magnitudes;
+  a.scales = w.scales;
+  a.const_m = w.const_m;
+  a.const_l = w.const_l;
+  a.const_p = w.const_p;
+  a.has_mask = has_mask;
+  a.batch = n;
+  a.n = n;
+  a.np = w.np;
+  return a;
+}
+
+// has_mask = 0: the prepare stage ran without a mask.
+int attend_stage(int dtype, int n, int has_mask, void* workspace, size_t workspace_bytes,
+                 void* stream) {
+  if (!block_dims_ok(n, fpx::kChannels, fpx::kHeads, fpx::kHeadDim, dtype)) return FPX_ERR_DIMS;
+  if (int rc = check_workspace(n, dtype, workspace, workspace_bytes)) return rc;
+  const BlockPointers w = block_pointers(workspace, n, dtype);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == FPX_BF16) {
+    fpx::Bf16AttnArgs a{};
+    a.q = as<__bf16>(w.qh);
+    a.k = as<__bf16>(w.kh);
+    a.v = as<__bf16>(w.vt);
+    a.mbias = w.mbias;
+    a.tile_flags = w.flags;
+    a.bias = as<__bf16>(w.tri);
+    a.gate = as<__bf16>(w.gs);
+    a.out = as<__bf16>(w.og);
+    a.batch = n;
+    a.n = n;
+    a.np = w.np;
+    return status(fpx::launch_attention_bf16(a, s));
+  }
+  return status(fpx::launch_attention_split(fpx::kAttnBlock,
+                                            block_attention_args(w, n, has_mask != 0), s));
+}
+
 // Output projection into dz, or added to dz (accumulate), in z's frame.
 int finish_stage(int dtype, const void* w_o, const void* b_o, int n, int ending, void* dz,
                  int64_t dz_stride0, int64_t dz_stride1, void* workspace, size_t workspace_bytes,
@@ -199,7 +252,7 @@ int block_impl(int dtype, const void* z, int64_t z_stride0, int64_t z_stride1, c
                                 ln_b, eps, w_qkvg, b_g, w_bias, mask_inf, n, ending, workspace,
                                 workspace_bytes, stream);
   if (rc) return rc;
-  rc = fpx_tri_attn_attend(dtype, n, workspace, workspace_bytes, stream);
+  rc = attend_stage(dtype, n, mask != nullptr, workspace, workspace_bytes, stream);
   if (rc) return rc;
   return finish_stage(dtype, w_o, b_o, n, ending, dz, dz_stride0, dz_stride1, workspace,
                       workspace_bytes, stream, accumulate);
@@ -401,52 +454,14 @@ int fpx_tri_attn_prepare(int dtype, const void* z, int64_t z_stride0, int64_t z_
   p.np = w.np;
   e = fpx::launch_projection(fpx::kProjBlock, p, s);
   if (e != hipSuccess) return status(e);
-  // the fast softmax reads the log2 bias relative to each query's reference
-  return status(fpx::launch_bias_reference(w.flags, n, n, w.np, p.tri_bias_l2, w.magnitudes, s));
+  // the fast softmax reads the log2 bias relative to each query's reference,
+  // constant-mask rows their shared weights
+  return status(fpx::launch_pair_bias(block_attention_args(w, n, mask != nullptr), p.tri_bias_l2,
+                                      w.magnitudes, w.flags, s));
 }
 
 int fpx_tri_attn_attend(int dtype, int n, void* workspace, size_t workspace_bytes, void* stream) {
-  if (!block_dims_ok(n, fpx::kChannels, fpx::kHeads, fpx::kHeadDim, dtype)) return FPX_ERR_DIMS;
-  if (int rc = check_workspace(n, dtype, workspace, workspace_bytes)) return rc;
-  const BlockPointers w = block_pointers(workspace, n, dtype);
-  const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == FPX_BF16) {
-    fpx::Bf16AttnArgs a{};
-    a.q = as<__bf16>(w.qh);
-    a.k = as<__bf16>(w.kh);
-    a.v = as<__bf16>(w.vt);
-    a.mbias = w.mbias;
-    a.tile_flags = w.flags;
-    a.bias = as<__bf16>(w.tri);
-    a.gate = as<__bf16>(w.gs);
-    a.out = as<__bf16>(w.og);
-    a.batch = n;
-    a.n = n;
-    a.np = w.np;
-    return status(fpx::launch_attention_bf16(a, s));
-  }
-  fpx::AttnArgs a{};
-  a.q = as<float>(w.qh);
-  a.k = as<float>(w.kh);
-  a.v = as<float>(w.vt);
-  a.mbias = w.mbias;
-  a.mb_stride = w.np;
-  a.bias = as<float>(w.tri);
-  a.bias_l2 = as<float>(w.tri) + (size_t)fpx::kHeads * w.np * w.np;
-  a.bias_stride = w.np;
-  a.bias_rows = w.np;
-  a.gate = as<float>(w.gs);
-  a.out = as<float>(w.og);
-  a.tile_flags = w.flags;
-  a.magnitudes = w.magnitudes;
-  a.scales = w.scales;
-  a.const_m = w.const_m;
-  a.const_l = w.const_l;
-  a.const_p = w.const_p;
-  a.batch = n;
-  a.n = n;
-  a.np = w.np;
-  return status(fpx::launch_attention_split(fpx::kAttnBlock, a, s));
+  return attend_stage(dtype, n, 1, workspace, workspace_bytes, stream);
 }
 
 int fpx_tri_attn_finish(int dtype, const void* w_o, const void* b_o, int n, int ending, void* dz,
@@ -616,7 +631,8 @@ int fpx_attn_strided(const float* q, int64_t q_sb, int64_t q_sh, int64_t q_sn, c
   void* kp = base + ws.kp;
   void* vp = base + ws.vp;
   float* scales = as<float>(base + ws.scales);
-  e = fpx::launch_stage_planes(a, qp, kp, vp, scales, as<float>(base + ws.partial), mag, st);
+  e = fpx::launch_stage_planes(a, qp, kp, vp, scales, as<float>(base + ws.partial), mag, flags,
+                               st);
   if (e != hipSuccess) return status(e);
   a.q = static_cast<const float*>(qp);
   a.k = static_cast<const float*>(kp);

@@ -10,6 +10,27 @@
 namespace fpx {
 namespace {
 
+// Zero rows [n, np) of every head of the triangle bias (padded queries), in
+// the FP32 or the BF16 fragment order, in each of `copies` consecutive
+// [4][np][np] copies (the FP32 block keeps the bias and its log2(e) copy);
+// work-group `group` of `groups` of 256 threads.
+template <typename BiasT>
+__device__ __forceinline__ void zero_bias_rows(int n, int np, BiasT* tri_bias, int copies,
+                                               int64_t group, int64_t groups) {
+  const int64_t per_head = (int64_t)(np - n) * np;
+  const int64_t total = kHeads * per_head;
+  const int64_t copy_elems = (int64_t)kHeads * np * np;
+  for (int64_t idx = group * 256 + threadIdx.x; idx < total; idx += groups * 256) {
+    const int h = (int)(idx / per_head);
+    const int64_t r = idx % per_head;
+    const int q = n + (int)(r / np);
+    const int k = (int)(r % np);
+    const int64_t at = sizeof(BiasT) == 4 ? bias_frag_index(h, q, k, np)
+                                          : bias_frag_index_bf16(h, q, k, np);
+    for (int c = 0; c < copies; ++c) tri_bias[c * copy_elems + at] = (BiasT)0.0f;
+  }
+}
+
 // One wavefront per row i < rows: mbias[i][k] for k < np and the row's tile
 // flags.  Word w of part 0 (the first kTileFlagWords words) has bit t % 32 of
 // tile t = 32w + t % 32 set when some key of that 32-key tile has a nonzero
@@ -22,13 +43,26 @@ namespace {
 // expression is (patches/protenix/0005-*.patch:36-39); otherwise the source
 // already holds mask-bias values and is copied.  np is a multiple of 64.
 // Work-group 0 also zeroes the magnitude record (nullable).
+// The work-groups past the rows' zero the padded query rows of the triangle
+// bias (tri_bias nullable; bias_bf16: its element type): one launch for both,
+// since at small N a launch costs more than either does.
 template <bool kFromMask>
 __global__ __launch_bounds__(256) void mask_rows_kernel(const float* __restrict__ mask,
                                                         int64_t ms_i, int64_t ms_j, int rows,
                                                         int n, int np, float inf,
                                                         float* __restrict__ mbias,
                                                         uint32_t* __restrict__ flags,
-                                                        uint32_t* __restrict__ magnitudes) {
+                                                        uint32_t* __restrict__ magnitudes,
+                                                        void* tri_bias, bool bias_bf16) {
+  const int row_groups = (rows + 3) / 4;
+  if ((int)blockIdx.x >= row_groups) {
+    const int64_t group = (int)blockIdx.x - row_groups, groups = (int)gridDim.x - row_groups;
+    if (bias_bf16)
+      zero_bias_rows(n, np, static_cast<__bf16*>(tri_bias), 1, group, groups);
+    else
+      zero_bias_rows(n, np, static_cast<float*>(tri_bias), 2, group, groups);
+    return;
+  }
   if (magnitudes != nullptr && blockIdx.x == 0 && threadIdx.x < kMagnitudeWords)
     magnitudes[threadIdx.x] = 0u;
   const int lane = threadIdx.x & 63;
@@ -70,26 +104,6 @@ __global__ __launch_bounds__(256) void mask_rows_kernel(const float* __restrict_
 #pragma unroll
     for (int wd = 0; wd < kTileFlagWords; ++wd)
       if (lane == pt * kTileFlagWords + wd) dst[pt * kTileFlagWords + wd] = part[pt][wd];
-}
-
-// Zero rows [n, np) of every head of the triangle bias (padded queries), in
-// the FP32 or the BF16 fragment order, in each of `copies` consecutive
-// [4][np][np] copies (the FP32 block keeps the bias and its log2(e) copy).
-template <typename BiasT>
-__global__ void bias_pad_kernel(int n, int np, BiasT* __restrict__ tri_bias, int copies) {
-  const int64_t per_head = (int64_t)(np - n) * np;
-  const int64_t total = kHeads * per_head;
-  const int64_t copy_elems = (int64_t)kHeads * np * np;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int h = (int)(idx / per_head);
-    const int64_t r = idx % per_head;
-    const int q = n + (int)(r / np);
-    const int k = (int)(r % np);
-    const int64_t at = sizeof(BiasT) == 4 ? bias_frag_index(h, q, k, np)
-                                          : bias_frag_index_bf16(h, q, k, np);
-    for (int c = 0; c < copies; ++c) tri_bias[c * copy_elems + at] = (BiasT)0.0f;
-  }
 }
 
 // Both fragment-order copies of a caller's [4][n][n] bias with any strides.
@@ -228,21 +242,13 @@ hipError_t launch_mask_bias(const float* mask, int64_t ms_i, int64_t ms_j, int n
                             bool bias_bf16, uint32_t* magnitudes, hipStream_t stream) {
   if (n <= 0) return hipSuccess;
   if (np % 64 || np > kTileFlagWords * 32 * 32) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(mask_rows_kernel<true>, dim3((uint32_t)((n + 3) / 4)), dim3(256), 0, stream,
-                     mask, ms_i, ms_j, n, n, np, inf, mbias, tile_flags, magnitudes);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || np == n) return e;
   const int64_t total = (int64_t)kHeads * (np - n) * np;
-  int64_t blocks = (total + 255) / 256;
+  int64_t pad_groups = (total + 255) / 256;
   const int64_t cap = (int64_t)device_cu_count() * 16;
-  if (blocks > cap) blocks = cap;
-  if (bias_bf16) {
-    hipLaunchKernelGGL(bias_pad_kernel<__bf16>, dim3((uint32_t)blocks), dim3(256), 0, stream, n,
-                       np, static_cast<__bf16*>(tri_bias), 1);
-  } else {
-    hipLaunchKernelGGL(bias_pad_kernel<float>, dim3((uint32_t)blocks), dim3(256), 0, stream, n,
-                       np, static_cast<float*>(tri_bias), 2);
-  }
+  if (pad_groups > cap) pad_groups = cap;
+  hipLaunchKernelGGL(mask_rows_kernel<true>, dim3((uint32_t)((n + 3) / 4 + pad_groups)), dim3(256),
+                     0, stream, mask, ms_i, ms_j, n, n, np, inf, mbias, tile_flags, magnitudes,
+                     tri_bias, bias_bf16);
   return hipGetLastError();
 }
 
@@ -252,7 +258,8 @@ hipError_t launch_mask_rows(const float* values, int64_t vs_i, int64_t vs_k, int
   if (rows <= 0 || n <= 0) return hipSuccess;
   if (np % 64 || np < n || np > kTileFlagWords * 32 * 32) return hipErrorInvalidValue;
   hipLaunchKernelGGL(mask_rows_kernel<false>, dim3((uint32_t)((rows + 3) / 4)), dim3(256), 0,
-                     stream, values, vs_i, vs_k, rows, n, np, 0.0f, mbias, tile_flags, magnitudes);
+                     stream, values, vs_i, vs_k, rows, n, np, 0.0f, mbias, tile_flags, magnitudes, nullptr,
+                     false);
   return hipGetLastError();
 }
 

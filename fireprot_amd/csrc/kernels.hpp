@@ -49,6 +49,12 @@ enum AttnLayout { kAttnBlock = 0, kAttnHeadLast = 1, kAttnStrided = 2, kAttnStag
 constexpr int kTileFlagWords = 4;
 constexpr int kTileFlagParts = 4;
 constexpr int kTileFlagMaxPart = 3;
+// Words 2 and 3 of part 3: the largest squared 2-norms of the row's q and k
+// vectors over its keys and heads (float bits, NaN-propagating), which bound
+// its products q.k by Cauchy-Schwarz.  Formed only on rows whose mask bias is
+// one finite nonzero value; zeroed by the mask stage.
+constexpr int kRowNormQ = 2;
+constexpr int kRowNormK = 3;
 
 // Per-tile exponent range of the fp16 planes: |e| <= kPlaneExpMax, so the
 // product scale 2^-(e_q + e_k) times log2(e) stays a normal float.
@@ -74,7 +80,7 @@ constexpr float kFastBound = 2097152.0f;  // 2^21
 // non-finite value disables the skip), then 1 once the projection wrote them.
 // A skipped key with a non-finite v would have made the native row NaN
 // (0 * inf), hence max|v| must be finite too.  Word kRelativeBiasWord is 1
-// when launch_bias_reference rewrote the log2-scaled bias copy relative to
+// when launch_pair_bias rewrote the log2-scaled bias copy relative to
 // each query's reference (zeroed with the rest of the record by the mask
 // stage).
 constexpr int kMagnitudeWords = 6;
@@ -105,17 +111,17 @@ struct AttnArgs {
   const uint32_t* magnitudes;  // kAttnBlock: nullable; enables the trailing-tile skip
   const float* scales;  // kAttnBlock, kAttnStaged: the planes' inverse scales
   // kAttnBlock, nullable: the constant-mask rows' shared weights and work
-  // lists, written by the split launch itself (const_weights_kernel):
-  // const_m[0] the mask bias m the weights serve (float bits; a NaN when no
-  // row has a constant mask), const_m[1] and const_m[2] the numbers of
-  // kConstRows-row chunks with constant-mask rows of that m and of another
-  // m, their chunk indices from word kConstListWord (the first list) and
-  // kConstListWord + ceil(batch / kConstRows) (the second);
-  // const_l[4][np] each query's weight sum, const_p the weights' fp16 planes,
-  // 4 KB per (head, 32-query tile, key tile).  Each may be null only with all.
+  // list, written by launch_pair_bias: const_m[0] the mask bias m the weights
+  // serve (float bits; a NaN when no row has a constant mask), const_m[1] and
+  // const_m[2] the numbers of kConstRows-row chunks with constant-mask rows
+  // of that m and of another m, the latter's chunk indices from word
+  // kConstListWord; const_l[4][np] each query's weight sum, const_p the
+  // weights' fp16 planes, 4 KB per (head, 32-query tile, key tile).  Each may
+  // be null only with all.
   uint32_t* const_m;
   float* const_l;
   uint8_t* const_p;
+  bool has_mask;  // kAttnBlock: the call has a mask (else every mask bias is 0)
   int64_t qs[3];  // kAttnStrided: (batch, head, row) element strides
   int64_t ks[3];
   int64_t vs[3];
@@ -131,21 +137,26 @@ struct AttnArgs {
 // for kAttnBlock or kAttnStaged.
 hipError_t launch_attention(int layout, const AttnArgs& args, hipStream_t stream);
 hipError_t launch_attention_split(int layout, const AttnArgs& args, hipStream_t stream);
-// The FP32 block after its prepare stage: rewrite bias_l2 ([4][np][np],
+// The FP32 block after its projection: rewrite bias_l2 ([4][np][np],
 // bias_frag_index order) as bias log2(e) - C_q + kRelOffset and set
 // magnitudes[kRelativeBiasWord] = 1, unless no key tile precedes every row's
-// first masked tile (then nothing changes).  flags: the rows' tile flags.
-hipError_t launch_bias_reference(const uint32_t* flags, int batch, int n, int np, float* bias_l2,
-                                 uint32_t* magnitudes, hipStream_t stream);
+// first masked tile (then nothing changes); with a mask (args.has_mask) form
+// the shared weights of the constant-mask rows and write their norms
+// (kRowNormQ, kRowNormK) to tile_flags (args.tile_flags, writable).  Reads
+// args' q, k, scales, bias, tile_flags, magnitudes, batch, n and np; writes
+// const_m, const_l, const_p.
+hipError_t launch_pair_bias(const AttnArgs& args, float* bias_l2, uint32_t* magnitudes,
+                            uint32_t* tile_flags, hipStream_t stream);
 // kAttnStrided q, k, v of args -> the plane layout of kAttnStaged: q_planes,
 // k_planes, v_planes each [batch][4] slices of np * 128 bytes, scales
 // [3][batch][4][np / 32] floats.
 // magnitudes (nullable, with partial of 3 stage_planes_groups floats):
 // words 0-2 of the record (max |q|, |k|, |v|) and word 4.
+// tile_flags (nullable): the rows' tile flags; receives kRowNormQ, kRowNormK.
 int64_t stage_planes_groups(const AttnArgs& args);
 hipError_t launch_stage_planes(const AttnArgs& args, void* q_planes, void* k_planes,
                                void* v_planes, float* scales, float* partial,
-                               uint32_t* magnitudes, hipStream_t stream);
+                               uint32_t* magnitudes, uint32_t* tile_flags, hipStream_t stream);
 
 // --------------------------------------------------------------- projection
 // Row tiles are 32 consecutive j of one outer row i; A rows are read at

@@ -147,6 +147,22 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
+// Whether outer row b's mask bias is one finite nonzero value m over its keys
+// (part 3 of the tile flags; false for NaN anywhere).
+__device__ __forceinline__ bool constant_mask(const uint32_t* tile_flags, int64_t b, float& m) {
+  const uint32_t* f = tile_flags + (b * kTileFlagParts + kTileFlagMaxPart) * kTileFlagWords;
+  const float lo = __builtin_bit_cast(float, f[1]);
+  m = __builtin_bit_cast(float, f[0]);
+  return m == lo && m != 0.f && __builtin_fabsf(m) < INFINITY;
+}
+// Raises row b's largest squared 2-norm of q (op 0) or k (op 1) to s >= 0
+// (or NaN, which sorts above infinity as unsigned bits).
+__device__ __forceinline__ void note_row_norm(uint32_t* tile_flags, int64_t b, int op, float s) {
+  atomicMax(tile_flags + (b * kTileFlagParts + kTileFlagMaxPart) * kTileFlagWords +
+                (op == 0 ? kRowNormQ : kRowNormK),
+            __builtin_bit_cast(uint32_t, s));
+}
+
 // Lane 0 of each 16-lane row, broadcast to the row (DPP row_newbcast:0).
 __device__ __forceinline__ float row16_first(float v) {
   return dpp<0x150>(v);
