@@ -13,8 +13,7 @@
 // incoming read of z^T goes through strides, with no transposed copy.
 //
 // Three launches:
-//   gated_split_kernel<kGatedTriMul>
-//                          LN_in, the four 128x128 projections, sigmoid gates
+//   gated_split_kernel     LN_in, the four 128x128 projections, sigmoid gates
 //                          and the mask; writes a and b channel-blocked (each
 //                          channel's rows as 32-key runs, gated_split.hpp)
 //                          with each (channel, row)'s max |value|
@@ -42,7 +41,7 @@ constexpr int kRows = 32;                 // pair rows per finish tile
 // the A and B row panels a range touches stay in that XCD's L2.
 // gemm_nt_128_f16 (16-bit matrix cores, scaled fp16 planes), with each row's
 // exponent from the row maxima the projection recorded, on the
-// channel-blocked a and b of gated_split_kernel<kGatedTriMul> (channel c's
+// channel-blocked a and b of gated_split_kernel (channel c's
 // row r at ((c / 16) np / 32 np + r) 512 + (c % 16) 32, rows 512 floats
 // apart, 32-key runs np * 512 floats apart).
 __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const float* __restrict__ pa,
@@ -75,7 +74,7 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const float* __
     const int64_t run = 512 * (int64_t)np;  // floats between a row's 32-key runs
     const int64_t cbase = (int64_t)(c >> 4) * (np / 32) * run + (c & 15) * 32;
     gemm_nt_128_f16(pa + cbase + 512 * (int64_t)i0, 512, pb + cbase + 512 * (int64_t)j0, 512,
-                    run, np / kSplitK, As, Bs, ea, eb, acc);
+                    run, (n + 31) / 32 * 32 / kSplitK, As, Bs, ea, eb, acc);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
 #pragma unroll
@@ -126,10 +125,15 @@ constexpr int kFinPlaneRow = kChannels + 8;  // bf16 per LDS row: 272 bytes
 
 __global__ __launch_bounds__(512, 1) void trimul_finish_split_kernel(TriMulArgs a, int tiles_j,
                                                                      int ntiles) {
-  __shared__ __attribute__((aligned(16))) __bf16 px[2][2][kRows][kFinPlaneRow];
-  __shared__ __attribute__((aligned(16))) __bf16 pz[2][2][kRows][kFinPlaneRow];
+  typedef __bf16 Planes[2][2][kRows][kFinPlaneRow];
+  __shared__ __attribute__((aligned(16))) Planes pxz[2];
+  Planes& px = pxz[0];
+  Planes& pz = pxz[1];
   __shared__ __attribute__((aligned(16))) float raw_x[kRows][kChannels + 4];
   __shared__ __attribute__((aligned(16))) float raw_z[kRows][kChannels + 4];
+  // the weights' way in (its 68 KB do not fit beside the planes)
+  float (*const turn)[kRowStage] = reinterpret_cast<float (*)[kRowStage]>(&pxz[0][0][0][0][0]);
+  static_assert(8 * kRowStage * sizeof(float) <= sizeof(pxz), "within the planes");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -140,49 +144,6 @@ __global__ __launch_bounds__(512, 1) void trimul_finish_split_kernel(TriMulArgs 
   const int n = a.n;
   const int64_t nb = a.np / 32;
   const bool residual = a.accumulate != 0;
-
-  // Weight planes: B[k][c] = W[c][k], lane holding keys 32t + 8 g4 + e, as
-  // fp16 (hi, lo) of W[c] 2^ew (each channel row's max |w| over the four
-  // lanes l16 + 16 g4 that hold it).
-  bf16x8 wz[2][4], wg[2][4];
-  int ewz, ewg;
-  {
-    f32x8 vz[4], vg[4];
-    float mz = 0.f, mg = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float* sz = a.w_z + (int64_t)ch * kChannels + 32 * t + 8 * g4;
-      const float* sg = a.w_g + (int64_t)ch * kChannels + 32 * t + 8 * g4;
-      const f32x4 z0 = *(const f32x4*)sz, z1 = *(const f32x4*)(sz + 4);
-      const f32x4 g0 = *(const f32x4*)sg, g1 = *(const f32x4*)(sg + 4);
-      vz[t] = f32x8{z0.x, z0.y, z0.z, z0.w, z1.x, z1.y, z1.z, z1.w};
-      vg[t] = f32x8{g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        mz = __builtin_elementwise_maximum(mz, __builtin_fabsf(vz[t][e]));
-        mg = __builtin_elementwise_maximum(mg, __builtin_fabsf(vg[t][e]));
-      }
-    }
-    auto rows4_max = [](float v) {  // lanes l, l ^ 16, l ^ 32, l ^ 48
-      const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
-                                                      __builtin_bit_cast(unsigned, v), false, false);
-      v = __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)s[0]),
-                                        __builtin_bit_cast(float, (unsigned)s[1]));
-      const auto u = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v),
-                                                      __builtin_bit_cast(unsigned, v), false, false);
-      return __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)u[0]),
-                                           __builtin_bit_cast(float, (unsigned)u[1]));
-    };
-    ewz = plane_exp(rows4_max(mz));
-    ewg = plane_exp(rows4_max(mg));
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      split_f16(ldexp8(vz[t], ewz), wz[0][t], wz[1][t]);
-      split_f16(ldexp8(vg[t], ewg), wg[0][t], wg[1][t]);
-    }
-  }
-  const float bz = a.b_z ? a.b_z[ch] : 0.f;
-  const float bg = a.b_g ? a.b_g[ch] : 0.f;
 
   // LN lanes: 16 per row, lane c16 = l16 holding channels 8 c16 .. +7 of
   // tile row lrow.
@@ -232,6 +193,59 @@ __global__ __launch_bounds__(512, 1) void trimul_finish_split_kernel(TriMulArgs 
     const f32x4 v = *(const f32x4*)(zr + 4);
     sz_raw = f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
   };
+  const int stride = (int)gridDim.x;
+  int tile = blockIdx.x;  // grid <= ntiles: every work-group has a tile
+  int next = tile + stride;
+  fetch(tile);  // in flight beside the weights
+
+  // Weight planes: B[k][c] = W[c][k], lane holding keys 32t + 8 g4 + e, as
+  // fp16 (hi, lo) of W[c] 2^ew (each channel row's max |w| over the four
+  // lanes l16 + 16 g4 that hold it).
+  bf16x8 wz[2][4], wg[2][4];
+  int ewz, ewg;
+  {
+    f32x8 vz[4], vg[4];
+    float mz = 0.f, mg = 0.f;
+    {
+      const Rows16 rz = fetch_rows16(a.w_z + (int64_t)16 * w * kChannels, lane);
+      const Rows16 rg = fetch_rows16(a.w_g + (int64_t)16 * w * kChannels, lane);
+      const float* src = turn[w] + l16 * kRowPad + 8 * g4;
+      put_rows16(rz, turn[w], lane);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vz[t] = *(const f32x8*)(src + 32 * t);
+      put_rows16(rg, turn[w], lane);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) vg[t] = *(const f32x8*)(src + 32 * t);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        mz = __builtin_elementwise_maximum(mz, __builtin_fabsf(vz[t][e]));
+        mg = __builtin_elementwise_maximum(mg, __builtin_fabsf(vg[t][e]));
+      }
+    }
+    auto rows4_max = [](float v) {  // lanes l, l ^ 16, l ^ 32, l ^ 48
+      const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
+                                                      __builtin_bit_cast(unsigned, v), false, false);
+      v = __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)s[0]),
+                                        __builtin_bit_cast(float, (unsigned)s[1]));
+      const auto u = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v),
+                                                      __builtin_bit_cast(unsigned, v), false, false);
+      return __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)u[0]),
+                                           __builtin_bit_cast(float, (unsigned)u[1]));
+    };
+    ewz = plane_exp(rows4_max(mz));
+    ewg = plane_exp(rows4_max(mg));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      split_f16(ldexp8(vz[t], ewz), wz[0][t], wz[1][t]);
+      split_f16(ldexp8(vg[t], ewg), wg[0][t], wg[1][t]);
+    }
+  }
+  const float bz = a.b_z ? a.b_z[ch] : 0.f;
+  const float bg = a.b_g ? a.b_g[ch] : 0.f;
+
   auto copy_raw = [&]() {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -339,14 +353,11 @@ __global__ __launch_bounds__(512, 1) void trimul_finish_split_kernel(TriMulArgs 
   };
 
   const bool lead = w < 4;
-  const int stride = (int)gridDim.x;
-  int tile = blockIdx.x;  // grid <= ntiles: every work-group has a tile
-  int next = tile + stride;
   {
     int i0, jb0;
     origin(tile, i0, jb0);
-    fetch(tile);
     copy_raw();
+    __syncthreads();  // every wave is past its weights' way in
     normalise(0, jb0 * kRows);
   }
   fetch(next);
@@ -411,7 +422,9 @@ hipError_t launch_trimul(const TriMulArgs& a, hipStream_t stream) {
     g.xs_k = a.outgoing ? a.zs_j : a.zs_i;
     g.rows_r = a.n;
     g.rows_k = a.n;
-    g.span_k = a.np;
+    // the contraction reads the keys of the tiles that hold any (< round_up(n, 32))
+    g.span_k = (a.n + kRows - 1) / kRows * kRows;
+    g.blocks_k = a.np / kRows;
     g.ln_w = a.ln_in_w;
     g.ln_b = a.ln_in_b;
     g.eps = a.eps_in;
@@ -428,8 +441,7 @@ hipError_t launch_trimul(const TriMulArgs& a, hipStream_t stream) {
     g.out[1] = a.pb;
     g.np = a.np;
     g.rowmax = a.rowmax;
-    if (a.rowmax == nullptr) return hipErrorInvalidValue;
-    e = launch_gated_split<kGatedTriMul>(g, stream);
+    e = launch_gated_split(g, stream);
   }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(trimul_contract_kernel, dim3((uint32_t)gemm_total), dim3(256), 0, stream,
