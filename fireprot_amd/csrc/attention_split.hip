@@ -373,6 +373,8 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, int nqt, int nkt_
   const int j0 = qt * kBq;
   const int jq = j0 + 32 * w + l32;
   const int qt32 = (j0 >> 5) + w;
+  // Queries past the tile that holds n - 1 have no planes: they run as zeros.
+  const bool live = j0 + 32 * w < a.n;  // uniform per wave
 
   // Per-work-group buffer descriptors over the (b, h) slices and the wave's
   // bias fragments (h, qt32, all key tiles), as in the FP32 kernel.
@@ -453,7 +455,7 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, int nqt, int nkt_
   {
     const int64_t per = (int64_t)kHeads * nt;
     const float* sc = a.scales + (int64_t)b * per + (int64_t)h * nt;
-    sq = sc[qt32];
+    if (live) sq = sc[qt32];
     float vmax = 0.f;
     for (int t = tid; t < nkt_all; t += kThreads) {
       if (t < nkt) Sk[t] = sc[(int64_t)a.batch * per + t];
@@ -494,8 +496,8 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, int nqt, int nkt_
     // Q planes, the B operand of S^T: lane holds Q[jq][16m + 8half + e], the
     // fp16 hi and lo planes (the log2(e) of the fast path enters with the
     // product scale).
-    bf16x8 qh[2], ql[2];
-    if (!kConst) {
+    bf16x8 qh[2] = {}, ql[2] = {};
+    if (!kConst && live) {
       const uint8_t* src = reinterpret_cast<const uint8_t*>(a.q) + bh * slice_bytes + (int64_t)jq * 64;
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
@@ -1215,7 +1217,7 @@ __device__ __forceinline__ void row_norms(const AttnArgs& a, uint32_t* tile_flag
     const uint8_t* src = reinterpret_cast<const uint8_t*>(op == 0 ? a.q : a.k) + bh * slice_bytes;
     float top = 0.f;
 #pragma unroll 4
-    for (int c = tid; c < 4 * a.np; c += kT) {
+    for (int c = tid; c < 4 * (int)round_up(a.n, 32); c += kT) {
       const f16x8 v = __builtin_bit_cast(f16x8, *(const bf16x8*)(src + (int64_t)c * 16));
       float s = 0.f;
 #pragma unroll

@@ -435,7 +435,9 @@ int fpx_tri_attn_prepare(int dtype, const void* z, int64_t z_stride0, int64_t z_
   p.xs_j = xs_j;
   p.rows_i = n;
   p.rows_j = n;
-  p.span_j = w.np;
+  // key and query tiles that hold a row; the attention reads none past them
+  // but for the queries of its last work-group, whose results it drops
+  p.span_j = (int)round_up(n, 32);
   p.ln_w = static_cast<const float*>(ln_w);
   p.ln_b = static_cast<const float*>(ln_b);
   p.eps = eps;

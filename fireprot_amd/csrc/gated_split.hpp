@@ -26,7 +26,7 @@
 // both normalising the tile, and its rows dealt over half as many streams:
 // 700 us at N = 1000, 48 at N = 256, 45 at N = 160; now 540, 43, 30.
 //
-// The pipeline is that of projection_split_kernel<kProjBlock>: LayerNorm 16
+// The pipeline is that of projection_block_kernel: LayerNorm 16
 // lanes per row, raw rows staged through LDS so that a row load is waited
 // an iteration after its issue, and lead / trail waves running the k steps
 // and the normalise-and-store half in opposite orders.
@@ -165,8 +165,9 @@ static __global__ __launch_bounds__(kGatedWaves * 64, 1) void gated_split_kernel
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     f32x8 wv[8];
-    rows32_operand(a.w_value[s] + (int64_t)16 * w * kChannels,
-                   a.w_gate[s] + (int64_t)16 * w * kChannels, turn[w], lane, wv);
+    rows32_operand(fetch_rows16(a.w_value[s] + (int64_t)16 * w * kChannels, lane),
+                   fetch_rows16(a.w_gate[s] + (int64_t)16 * w * kChannels, lane), turn[w], lane,
+                   wv);
     float m = 0.f;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -217,17 +218,24 @@ static __global__ __launch_bounds__(kGatedWaves * 64, 1) void gated_split_kernel
   // Both slices' products of a tile, scaled back.
   auto k_steps = [&](int buf, f32x16 (&res)[2]) {
     f32x16 c0 = {}, c1 = {};
+    // The small terms hi lo and lo hi are summed first, so a chain rounds at
+    // the size of the result eight times and not at all 24 steps.
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       const int k = 16 * t + 8 * half;
       const bf16x8 xh = *(const bf16x8*)&xs[buf][0][l32][k];
       const bf16x8 xl = *(const bf16x8*)&xs[buf][1][l32][k];
-      c0 = mfma_f16(xh, wh[0][t], c0);
-      c1 = mfma_f16(xh, wh[1][t], c1);
       c0 = mfma_f16(xh, wl[0][t], c0);
       c1 = mfma_f16(xh, wl[1][t], c1);
       c0 = mfma_f16(xl, wh[0][t], c0);
       c1 = mfma_f16(xl, wh[1][t], c1);
+    }
+    asm volatile("" ::: "memory");  // the hi plane is read again, not kept in 32 registers
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const bf16x8 xh = *(const bf16x8*)&xs[buf][0][l32][16 * t + 8 * half];
+      c0 = mfma_f16(xh, wh[0][t], c0);
+      c1 = mfma_f16(xh, wh[1][t], c1);
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -325,7 +333,7 @@ static __global__ __launch_bounds__(kGatedWaves * 64, 1) void gated_split_kernel
     if (lead) k_steps(buf, res);
     {
       // The other half: normalise T_{k+1} into the other planes, then the
-      // iteration's global accesses (see projection_split_kernel).
+      // iteration's global accesses (see projection_block_kernel).
       const bool more = i + 1 < count;
       if (more) {
         int rn, kn0;

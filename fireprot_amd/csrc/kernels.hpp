@@ -174,7 +174,7 @@ struct ProjArgs {
   int64_t xs_j;
   int rows_i;
   int rows_j;    // valid j extent
-  int span_j;    // j extent covered by tiles (np for kProjBlock, else rows_j)
+  int span_j;    // j extent covered by tiles (rows_j, kProjBlock: rounded up to 32)
   const float* ln_w;
   const float* ln_b;
   float eps;

@@ -167,9 +167,8 @@ __device__ __forceinline__ void put_rows16(const Rows16& r, float* lds, int lane
 }
 // 32 rows (two runs of 16) as the B operand of the 32x32x16 products: lane
 // (l32, half) gets channels 16 t + 8 half + e of row l32 in wv[t][e].
-__device__ __forceinline__ void rows32_operand(const float* lo16, const float* hi16, float* lds,
+__device__ __forceinline__ void rows32_operand(const Rows16& a, const Rows16& b, float* lds,
                                                int lane, f32x8 (&wv)[8]) {
-  const Rows16 a = fetch_rows16(lo16, lane), b = fetch_rows16(hi16, lane);
   const float* src = lds + (lane & 15) * kRowPad + 8 * (lane >> 5);
   const bool upper = (lane >> 4) & 1;
   put_rows16(a, lds, lane);
