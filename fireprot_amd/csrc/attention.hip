@@ -1,59 +1,60 @@
-// Flash-style triangle attention on the CDNA4 FP32 matrix cores, on the
-// reference C-ABI layout (q, k, v, out [B][n][4][32], a shared [4][n][S]
-// bias): the kernel behind ck_attention, ck_attention_exact1536,
-// ck_attention_vector_bias1000, fpx_attn_core and fpx_attn_core_masked.
-// The block and the strided (OpenFold3) entries run attention_split_kernel.
+// Flash-style triangle attention on the reference C-ABI layout (q, k, v, out
+// [B][n][4][32], a shared [4][n][S] bias): the kernel behind ck_attention,
+// ck_attention_exact1536, ck_attention_vector_bias1000, fpx_attn_core and
+// fpx_attn_core_masked.  The block and the strided (OpenFold3) entries run
+// attention_split_kernel on planes staged in a workspace; these entries have
+// none, so this kernel splits its operands as it goes.
 //
 // One work-group = (outer row b, head h, 128 queries); four wavefronts, each
-// owning 32 queries.  Keys are streamed in tiles of 32.  K and V^T tiles are
-// staged once in LDS for the four waves, in double buffers, so there is one
-// barrier per tile.  The N x N logits of a row and the N^3 score volume never
-// reach HBM.
+// owning 32 queries.  Keys are streamed in tiles of 32.  Both products run on
+// v_mfma_f32_32x32x16_f16 with power-of-two scaled fp16 (hi, lo) planes and
+// three terms (FP32 accuracy, split.hpp).  Per tile the four waves load its K
+// and V rows two tiles ahead, find the tile's largest |K| and |V| one tile
+// ahead, and split them into planes in LDS (double-buffered, one barrier per
+// tile), each value once for the work-group's 128 queries:
+//   - q by 2^e_q (each wave's 32 queries), K by 2^e_k (each tile);
+//   - V by 2^E, E the smallest plane exponent of the tiles so far, so the
+//     weights of all tiles enter P.V at one scale; when a tile lowers E, O is
+//     scaled by the exact power of two between.
+// S^T = K Q^T and O^T += V^T P^T are transposed, so each lane column (lane %
+// 32) holds one query in both results: row statistics, the P operand and the
+// O rescale live in the lane that needs them, and the only cross-lane step is
+// an xor-32 exchange of a tile max.
 //
-// Per key tile each wave computes S^T = K Q^T (16 x v_mfma_f32_32x32x2_f32)
-// and O^T += V^T P^T (16 more).  With the transposed products, each lane
-// column (lane % 32) holds one query in both results.  The online-softmax row
-// statistics, the P operand and the O rescale therefore all live in the lane
-// that needs them.  The only cross-lane step is an xor-32 exchange of a tile
-// max.
+// The bias comes as rows of [n][S]: a wave's 32 x 32 fragment is copied by
+// global_load_lds as eight rows of 128 contiguous bytes per instruction into
+// 4 KB of LDS of its own and read back in accumulator order.  Loaded straight
+// into accumulator order, each instruction touches 32 rows.
 //
-// Cost model.  On gfx950 an FP32 MFMA and VALU work never overlap, whether
-// they come from one wave or from several waves of a SIMD: a tile costs its
-// 32 x 64 matrix cycles plus every VALU instruction around them, and a
-// v_exp_f32 costs about as much as three other VALU instructions while the
-// matrix cores are busy.  Software pipelining inside a wave buys nothing but
-// load slack, so each tile runs S^T, softmax and O^T += V^T P^T in order, and
-// the loop is built to issue as few VALU instructions as possible.
+// Rows with at least one unmasked key (fast): logits fma(acc, 2^-(e_q+e_k),
+// bias) in natural units (plus the mask bias on masked tiles), weights
+// P' = exp2(fma(x, log2(e), -c)) with one integer reference c per query, 7
+// below the ceiling of the largest logit when it was set: no max is formed
+// until a lane's 16 weights of a tile sum past 2^15 (or at the first tile).
+// A masked key of such a row gets weight exactly 0 whatever the rounding of
+// its logit, because its logit is about -1e9 below the row max.
 //
-// Rows with at least one unmasked key (the fast path):
-//   - S^T accumulates from zero and one fma per logit adds the triangle
-//     bias pre-scaled by log2(e) (loaded from a fragment-major copy straight
-//     into registers): fma(s, log2(e), bias log2(e)), logits in log2 units.
-//     The dot product's partial sums thus round at its own magnitude; with
-//     the bias as the accumulator's start value they rounded at the bias's
-//     (|logit| ~ 60 in log2 units), about ten times the error of FP32
-//     native attention.
-//   - The mask bias is added only on tiles flagged as masked.  A masked key
-//     of such a row gets weight exactly 0 whatever the rounding of its logit,
-//     because its logit is about -1e9 below the row max.
-//   - Weights are exp2(x - c) with one reference c per query, and c = 0
-//     whenever the row max lies within 2^+-56.  Then a tile needs neither a
-//     max nor a subtraction: 16 exp2 and the adds of the row sum.  A tile max
-//     is formed only for the first tile and when the running sum passes
-//     2^64; O and l are then rescaled to the new reference.
-// Rows whose keys are all masked (the exact path):
-//   - Every tile forms fl(fl(s + mask_bias) + bias) in natural units, the
-//     native order (patches/protenix/0005-*.patch:36-45; kernels/amd/
-//     fireprot_softmax_fp32.cpp:33-35), from the unscaled q and an unscaled
-//     bias copy.  These logits are quantised to the FP32 spacing of -1e9 (64),
-//     and this order reproduces which keys tie at the max.  Weights are
-//     exp2(fma(x, log2 e, -c)) with c = fl(m log2 e) of a lazy running max m
-//     (rescaled when a tile max exceeds it by 2^8), so equal logits get equal
-//     weights.
-// A row whose logits are all -inf gives NaN, as torch.softmax does.
+// Rows whose keys are all masked (exact): fl(fl(s + mask_bias) + bias) in
+// natural units, the native order (patches/protenix/0005-*.patch:36-45;
+// kernels/amd/fireprot_softmax_fp32.cpp:33-35).  These logits are quantised to
+// the FP32 spacing of -1e9 (64), and this order reproduces which keys tie at
+// the max.  Weights are exp2(fma(x, log2 e, -c)) with c = fl(m log2 e) of a
+// lazy running max m (rescaled when a tile max exceeds it by 2^8), so equal
+// logits get equal weights.
+//
+// A row whose logits are all -inf gives NaN, as torch.softmax does.  fp16
+// planes cannot carry an infinity beside finite values (its residual is NaN),
+// so a work-group that meets a non-finite q, k or v computes its rows in plain
+// FP32 (attend_scalar) with the native propagation.
+//
+// Bound: VALU issue beside the matrix cores (about 170 VALU instructions and
+// 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.23 ms; on the FP32
+// matrix cores, which never overlap with VALU work, 5.42 ms.  N = 384 175 us
+// against 287.
 #include "attn_common.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "split.hpp"
 
 #include <cmath>
 #include <type_traits>
@@ -61,330 +62,429 @@
 namespace fpx {
 namespace {
 
-constexpr int kPad = 4;    // LDS row padding (floats): conflict-free b128 reads
 constexpr int kThreads = 256;
-// Occupancy the register budget is set for (waves per SIMD).
-#ifndef FPX_ATTN_WAVES_PER_SIMD
-#define FPX_ATTN_WAVES_PER_SIMD 3
-#endif
+constexpr int kPlaneBytes = 2048;              // 32 rows of 64 bytes
+constexpr int kTileBytes = 4 * kPlaneBytes;    // K hi, K lo, V^T hi, V^T lo
+constexpr int kBiasBytes = 32 * kBk * 4;       // a wave's bias fragment
+constexpr float kPlaneMax = 32768.0f;          // bound on a lane's 16 scaled weights
+constexpr float kShift = 7.0f;                 // weights enter P.V as up to 2^7 and more
+constexpr int64_t kMaxBiasStride = 1 << 25;    // 31 rows within 32-bit byte offsets
+constexpr float kBigLogit = 4194304.0f;        // 2^22: past it, references take no shift
 
-typedef float KTile[kBk][kHeadDim + kPad];  // [key][channel]
-typedef float VTile[kHeadDim][kBk + kPad];  // [channel][key]
-
-// Tile sources of one work-group.  Every tile index passed in is in range.
-template <int LAYOUT>
-struct Tiles;
-
-// The reference C-ABI layout (kernels/amd/fireprot_ck_attention.cpp:34-43):
-// q, k, v, out [B][n][H][32]; bias [H][n][bias_stride]; mask bias nullable.
-template <>
-struct Tiles<kAttnHeadLast> {
-  const AttnArgs& a;
-  int b, h, row8, col4, half, jq;
-  __device__ __forceinline__ Tiles(const AttnArgs& args, int b_, int h_, int /*qt32*/, int tid,
-                                   int /*lane*/, int half_, int jq_)
-      : a(args), b(b_), h(h_), row8(tid >> 3), col4((tid & 7) * 4), half(half_), jq(jq_) {}
-  __device__ __forceinline__ f32x4 row(const float* base, int t) const {
-    const int key = t * kBk + row8;
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    return key < a.n
-               ? *(const f32x4*)(base + (((int64_t)b * a.n + key) * kHeads + h) * kHeadDim + col4)
-               : zero;
-  }
-  // thread (row8 = key, col4 = channel group) for both K and V
-  __device__ __forceinline__ f32x4 k(int t) const { return row(a.k, t); }
-  __device__ __forceinline__ f32x4 v(int t) const { return row(a.v, t); }
-  static __device__ __forceinline__ void store_v(VTile& vs, f32x4 v, int row8, int col4) {
-    vs[col4 + 0][row8] = v.x;
-    vs[col4 + 1][row8] = v.y;
-    vs[col4 + 2][row8] = v.z;
-    vs[col4 + 3][row8] = v.w;
-  }
-  __device__ __forceinline__ f32x16 bias(int t) const {
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 x[4];
+// The rows of this lane's query in plain FP32, two passes over the keys: for
+// work-groups with a non-finite operand, and for bias rows so far apart that
+// a wave's 32 span more than 4 GB.  Lane half `half` holds channels
+// 16 half .. + 15 of the query and of the output.
+__device__ __forceinline__ void attend_scalar(const AttnArgs& a, int b, int h, int jq, int half) {
+  const bool ok = jq < a.n;
+  const int64_t row = ((int64_t)b * a.n + (ok ? jq : 0)) * kHeads + h;
+  float q[16], o[16];
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int key = t * kBk + 8 * rr + 4 * half;  // n % 4 == 0: all-in or all-out
-      x[rr] = (jq < a.n && key < a.n)
-                  ? *(const f32x4*)(a.bias + ((int64_t)h * a.bias_rows + jq) * a.bias_stride + key)
-                  : zero;
-    }
-    return cat4(x[0], x[1], x[2], x[3]);
+  for (int i = 0; i < 16; ++i) {
+    q[i] = a.q[row * kHeadDim + 16 * half + i];
+    o[i] = 0.f;
   }
-  __device__ __forceinline__ f32x16 bias_l2(int t) const {
-    f32x16 r = bias(t);
+  const float* bias = a.bias + ((int64_t)h * a.bias_rows + (ok ? jq : 0)) * a.bias_stride;
+  auto logit = [&](int key) -> float {
+    const float* k = a.k + (((int64_t)b * a.n + key) * kHeads + h) * kHeadDim + 16 * half;
+    float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) r[i] *= kLog2e;
-    return r;
+    for (int i = 0; i < 16; ++i) s = __builtin_fmaf(q[i], k[i], s);
+    s = xor32_sum(s);
+    const float m = a.mbias ? a.mbias[(int64_t)b * a.mb_stride + key] : 0.f;
+    return (s + m) + bias[key];
+  };
+  float m = -INFINITY;
+#pragma unroll 1
+  for (int key = 0; key < a.n; ++key) m = __builtin_elementwise_maximum(m, logit(key));
+  float l = 0.f;
+#pragma unroll 1
+  for (int key = 0; key < a.n; ++key) {
+    const float p = exp2_fast((logit(key) - m) * kLog2e);
+    l += p;
+    const float* v = a.v + (((int64_t)b * a.n + key) * kHeads + h) * kHeadDim + 16 * half;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[i] = __builtin_fmaf(p, v[i], o[i]);
   }
-  __device__ __forceinline__ f32x16 mask(int t) const {
-    f32x16 r;
+  if (!ok) return;
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int key = t * kBk + 8 * rr + 4 * half + e;
-        r[4 * rr + e] = key < a.n ? (a.mbias ? a.mbias[(int64_t)b * a.mb_stride + key] : 0.f)
-                                  : -INFINITY;
-      }
-    }
-    return r;
-  }
-};
-
-// S^T[key][q] = c + sum_ch K[key][ch] Q[q][ch] for the 32 keys of ks; lane
-// half hb supplies channel 16*hb + s at step s.
-__device__ __forceinline__ f32x16 qk_chain(const KTile& ks, const float* qf, int l32, int half,
-                                           f32x16 c) {
-  f32x16 s = c;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const f32x4 kv = *(const f32x4*)&ks[l32][16 * half + 4 * t];
-    s = mfma32(kv.x, qf[4 * t + 0], s);
-    s = mfma32(kv.y, qf[4 * t + 1], s);
-    s = mfma32(kv.z, qf[4 * t + 2], s);
-    s = mfma32(kv.w, qf[4 * t + 3], s);
-  }
-  return s;
+  for (int i = 0; i < 16; ++i) a.out[row * kHeadDim + 16 * half + i] = o[i] / l;
 }
 
-template <int LAYOUT>
-__global__ __launch_bounds__(kThreads, FPX_ATTN_WAVES_PER_SIMD) void attention_kernel(
-    AttnArgs a, int nqt, int nkt, uint32_t total) {
-  static_assert(LAYOUT == kAttnHeadLast, "the reference C-ABI layout only");
-  __shared__ __attribute__((aligned(16))) KTile Ks[2];
-  __shared__ __attribute__((aligned(16))) VTile Vs[2];
+__global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int nqt, int nkt,
+                                                                uint32_t total, int ppg) {
+  __shared__ __attribute__((aligned(16))) uint8_t kv[2][kTileBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t bias_lds[kThreads / 64][kBiasBytes];
+  // each wave's largest |K| and |V| of tile t at [t & 1]; [2]: its largest |q|
+  __shared__ float red[3][kThreads / 64][2];
 
-  // Logical order, slowest to fastest: head, block of kRowGroup outer rows,
-  // query tile, outer row in the block.  The work-groups that run together
-  // on one XCD then share each triangle-bias slice across kRowGroup outer rows
-  // and each K/V slice across all query tiles, in that XCD's L2.
-  const uint32_t logical = xcd_remap(blockIdx.x, total);
-  const int groups = (a.batch + kRowGroup - 1) / kRowGroup;
-  const int per_head = groups * kRowGroup * nqt;
-  const int h = (int)(logical / per_head);
-  const int rem = (int)(logical % per_head);
-  const int grp = rem / (kRowGroup * nqt);
-  const int in_grp = rem % (kRowGroup * nqt);
-  const int qt = in_grp / kRowGroup;
-  const int b = grp * kRowGroup + in_grp % kRowGroup;
+  int b, h, qt;
+  attn_item(blockIdx.x, total, a.batch, nqt, ppg, b, h, qt);
   if (b >= a.batch) return;  // padding of the last row group; uniform per work-group
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
   const int l32 = lane & 31;
-  const int j0 = qt * kBq;
-  const int jq = j0 + 32 * w + l32;
-  const int qt32 = (j0 >> 5) + w;
-  const int row8 = tid >> 3;
-  const int col4 = (tid & 7) * 4;
+  const int j0 = qt * kBq + 32 * w;
+  const int jq = j0 + l32;
   const int last = nkt - 1;
-  const Tiles<LAYOUT> io(a, b, h, qt32, tid, lane, half, jq);
 
-  // Row classification.  masked(t): some key of tile t has a nonzero mask
-  // bias.  has_unmasked: some key k < n of the row has a zero mask bias.
-  const bool any_masked = a.mbias != nullptr || a.n % kBk != 0;
-  int found = a.mbias == nullptr;
-  if (!found) {
-    for (int k = tid; k < a.n; k += kThreads) found |= a.mbias[(int64_t)b * a.mb_stride + k] == 0.0f;
-  }
-  const bool has_unmasked = __syncthreads_or(found) != 0;
-  auto masked = [&](int t) -> bool {
-    return any_masked && (a.mbias != nullptr || (t + 1) * kBk > a.n);
-  };
-  auto mask_vals = [&](int t) -> f32x16 { return io.mask(t); };
+  // The planes path; false (uniform) when the rows need attend_scalar.
+  auto attend = [&]() -> bool {
+    if (a.bias_stride > kMaxBiasStride) return false;
 
-  // Q fragment (B operand of S^T = K Q^T): lane holds Q[jq][16*half + s].
-  float qf[16];
-  {
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const bool ok = jq < a.n;
-    const float* src = a.q + (((int64_t)b * a.n + (ok ? jq : 0)) * kHeads + h) * kHeadDim + 16 * half;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const f32x4 v = ok ? *(const f32x4*)(src + 4 * t) : zero;
-      qf[4 * t + 0] = v.x;
-      qf[4 * t + 1] = v.y;
-      qf[4 * t + 2] = v.z;
-      qf[4 * t + 3] = v.w;
+    // Row classification.  masked(t): some key of tile t has a nonzero mask
+    // bias.  has_unmasked: some key k < n of the row has a zero mask bias.
+    int found = a.mbias == nullptr;
+    if (!found) {
+      for (int k = tid; k < a.n; k += kThreads) found |= a.mbias[(int64_t)b * a.mb_stride + k] == 0.0f;
     }
-  }
-
-  f32x16 o = {};
-  float l_run = 0.f;
-
-  // O^T[c][q] += V^T[c][key] P^T[key][q]; lane register r of p is key
-  // 8*(r/4) + 4*half + r%4, as in the S^T accumulator.
-  auto pv = [&](const VTile& vs, const f32x16& p) {
+    const bool has_unmasked = __syncthreads_or(found) != 0;
+    auto masked = [&](int t) -> bool { return a.mbias != nullptr || (t + 1) * kBk > a.n; };
+    // f(r, mask bias of register r's key) over a tile, four registers at a time
+    // (all sixteen values at once would not fit the register budget).
+    auto with_mask = [&](int t, auto&& f) {
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const f32x4 vv = *(const f32x4*)&vs[l32][8 * rr + 4 * half];
-      o = mfma32(vv.x, p[4 * rr + 0], o);
-      o = mfma32(vv.y, p[4 * rr + 1], o);
-      o = mfma32(vv.z, p[4 * rr + 2], o);
-      o = mfma32(vv.w, p[4 * rr + 3], o);
-    }
-  };
-
-  // One pass over the key tiles.  Two register sets alternate between even
-  // and odd tiles: a tile's bias is loaded into its set two tiles ahead, the
-  // S^T chain of the tile accumulates there, and the weights go to p.
-  auto run = [&](auto exact_tag) {
-    constexpr bool kExact = decltype(exact_tag)::value;
-    const f32x16 zero16 = {};
-    f32x16 p;
-
-    // Reference state of this lane's query.
-    //   exact: m_ref = lazy running max (logit units), m_thr = the tile max
-    //     that triggers a rescale, c_ref = fl(m_ref log2 e) (0 while m_ref is
-    //     -inf, so all-(-inf) tiles give weight exp2(-inf) = 0).
-    //   fast: m_ref = largest tile max seen on the rare path (log2 units;
-    //     -inf while the query has no reference), c_ref = the reference;
-    //     has_ref / c_zero are wave-uniform.
-    float m_ref = -INFINITY;
-    float m_thr = -INFINITY;
-    float c_ref = 0.f;
-    bool has_ref = false;
-    bool c_zero = true;
-
-    // x: this tile's logits (exact: logit units; fast: log2 units) -> p.
-    auto softmax = [&](const f32x16& x) {
-      if (kExact) {
-        const float mt = xor32_max(max16(x));
-        if (__any(mt > m_thr)) {
-          const float m_new = __builtin_elementwise_maximum(m_ref, mt);
-          const float c_new = m_new == -INFINITY ? 0.f : m_new * kLog2e;
-          const float alpha = m_ref == -INFINITY ? 0.f : exp2_fast(c_ref - c_new);
+      for (int rr = 0; rr < 4; ++rr) {
+        float m[4];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[r] *= alpha;
-          l_run *= alpha;
-          m_ref = m_new;
-          c_ref = c_new;
-          m_thr = m_new + kRescaleNat;
+        for (int e = 0; e < 4; ++e) {
+          const int key = t * kBk + 8 * rr + 4 * half + e;
+          m[e] = key < a.n ? (a.mbias ? a.mbias[(int64_t)b * a.mb_stride + key] : 0.f) : -INFINITY;
         }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) p[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref));
-        l_run += sum16(p);
-        return;
+        for (int e = 0; e < 4; ++e) f(4 * rr + e, m[e]);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
       }
-      float ovf = 0.f;
-      if (has_ref) {
-        if (c_zero) {
+    };
+
+    // K rows: thread (key tid / 8, channels 4 (tid % 8) .. + 3).  V: thread
+    // (channel tid % 32, keys 4 (tid / 32) .. + 3), so its four keys are
+    // adjacent in the V^T planes.  Keys past n are loaded from the last key
+    // (no branch around the loads) and zeroed.
+    const int kkey = tid >> 3, kc4 = (tid & 7) * 4;
+    const int vc = tid & 31, vg = tid >> 5;
+    const float* const krow = a.k + ((int64_t)b * a.n * kHeads + h) * kHeadDim;
+    const float* const vrow = a.v + ((int64_t)b * a.n * kHeads + h) * kHeadDim;
+    auto load_kv = [&](int t, f32x4& kx, f32x4& vx) {
+      const int key = t * kBk + kkey;
+      kx = *(const f32x4*)(krow + (uint32_t)(min(key, a.n - 1) * kHidden + kc4));
 #pragma unroll
-          for (int r = 0; r < 16; ++r) p[r] = exp2_fast(x[r]);
+      for (int i = 0; i < 4; ++i)
+        vx[i] = vrow[(uint32_t)(min(t * kBk + 4 * vg + i, a.n - 1) * kHidden + vc)];
+    };
+    auto clip_kv = [&](int t, f32x4& kx, f32x4& vx) {  // uniform branch: the last tile at most
+      if ((t + 1) * kBk <= a.n) return;
+      if (t * kBk + kkey >= a.n) kx = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (t * kBk + 4 * vg + i >= a.n) vx[i] = 0.f;
+    };
+    auto max4 = [](const f32x4& x) -> float {
+      return __builtin_elementwise_maximum(
+          __builtin_elementwise_maximum(__builtin_fabsf(x.x), __builtin_fabsf(x.y)),
+          __builtin_elementwise_maximum(__builtin_fabsf(x.z), __builtin_fabsf(x.w)));
+    };
+    auto note_max = [&](const f32x4& kx, const f32x4& vx, int slot) {
+      const float mk = wave_max(max4(kx)), mv = wave_max(max4(vx));
+      if (lane == 0) {
+        red[slot][w][0] = mk;
+        red[slot][w][1] = mv;
+      }
+    };
+    auto read_max = [&](int slot, float& mk, float& mv) {
+      mk = red[slot][0][0];
+      mv = red[slot][0][1];
+#pragma unroll
+      for (int i = 1; i < kThreads / 64; ++i) {
+        mk = __builtin_elementwise_maximum(mk, red[slot][i][0]);
+        mv = __builtin_elementwise_maximum(mv, red[slot][i][1]);
+      }
+    };
+    // A staged tile into planes: 16-byte chunk c of a plane's row r sits at
+    // chunk c ^ swz(r).  V^T keys lie in the order of the S^T accumulator
+    // registers: key group g of four at position 16 (g / 4) + 4 (0, 2, 1,
+    // 3)[g % 4].
+    const uint32_t kput = kkey * 64 + 16 * ((kc4 >> 3) ^ swz(kkey)) + (kc4 & 4) * 2;
+    const int vpos = (vg >> 2) * 16 + ((vg & 1) * 2 + ((vg >> 1) & 1)) * 4;
+    const uint32_t vput = vc * 64 + 16 * ((vpos >> 3) ^ swz(vc)) + (vpos & 7) * 2;
+    auto put = [&](int stage, const f32x4& kx, const f32x4& vx, int ek, int ev) {
+      bf16x4 hi, lo;
+      split_f16(ldexp4(kx, ek), hi, lo);
+      *(bf16x4*)(kv[stage] + kput) = hi;
+      *(bf16x4*)(kv[stage] + kPlaneBytes + kput) = lo;
+      split_f16(ldexp4(vx, ev), hi, lo);
+      *(bf16x4*)(kv[stage] + 2 * kPlaneBytes + vput) = hi;
+      *(bf16x4*)(kv[stage] + 3 * kPlaneBytes + vput) = lo;
+    };
+    // plane_exp of a zero tile must not lower the smallest exponent
+    auto value_exp = [](float m) -> int {
+      return __builtin_amdgcn_readfirstlane(m == 0.f ? 141 : plane_exp(m));
+    };
+    auto plane_rd = [&](int stage, int plane, int m) -> bf16x8 {
+      return *(const bf16x8*)(kv[stage] + plane * kPlaneBytes + l32 * 64 +
+                              16 * ((2 * m + half) ^ swz(l32)));
+    };
+
+    // Bias fragment of tile t: instruction i copies rows 8 i + lane / 8 of the
+    // wave's 32 queries, 16-byte chunk lane % 8 from that row's chunk
+    // (lane % 8) ^ (lane / 8), so the reads in accumulator order are spread over
+    // the banks.  Rows past n are row n - 1, keys past n the row's last four:
+    // their queries are dropped, their logits masked.
+    const int chunk = (lane & 7) ^ (lane >> 3);
+    const int jw = min(j0, a.n - 1);  // the wave's first row
+    const uint64_t bits =
+        (uint64_t)(a.bias + ((int64_t)h * a.bias_rows + jw) * a.bias_stride);
+    const uint8_t* const brow = reinterpret_cast<const uint8_t*>(
+        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32) |
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)bits));
+    const uint32_t step = 8u * (uint32_t)a.bias_stride * 4u;
+    const int rows_left = a.n - 1 - jw;
+    const uint32_t bias_at = __builtin_amdgcn_readfirstlane((int)lds_address(bias_lds[w]));
+    auto bias_dma = [&](int t) {
+      const uint32_t col = 4u * (uint32_t)min(4 * chunk, a.n - 4 - t * kBk);
+      const uint8_t* base = brow + (int64_t)t * kBk * 4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t row = (uint32_t)min(8 * i + (lane >> 3), rows_left);
+        lds_dma16_s(row * (step >> 3) + col, base, bias_at + 1024 * i);
+      }
+    };
+    auto bias_rd = [&]() -> f32x16 {
+      const uint8_t* src = bias_lds[w] + l32 * 128;
+      f32x4 x[4];
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) x[rr] = *(const f32x4*)(src + 16 * ((2 * rr + half) ^ (l32 & 7)));
+      return cat4(x[0], x[1], x[2], x[3]);
+    };
+
+    // Q planes (B operand of S^T = K Q^T): lane holds Q[jq][16 m + 8 half + e].
+    bf16x8 qh[2], ql[2];
+    int eq, ek, ev;  // plane exponents of the wave's q, of the tile's K, and E
+    f32x4 ka, va;
+    {
+      const float* src = a.q + (((int64_t)b * a.n + min(jq, a.n - 1)) * kHeads + h) * kHeadDim + 8 * half;
+      f32x4 x[4];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        x[2 * m] = *(const f32x4*)(src + 16 * m);
+        x[2 * m + 1] = *(const f32x4*)(src + 16 * m + 4);
+      }
+      f32x4 k0, v0;
+      load_kv(0, k0, v0);
+      load_kv(last < 1 ? last : 1, ka, va);
+      bias_dma(0);
+      float mq = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mq = __builtin_elementwise_maximum(mq, max4(x[i]));
+      mq = wave_max(mq);
+      eq = __builtin_amdgcn_readfirstlane(plane_exp(mq));
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const f32x4 u = ldexp4(x[2 * m], eq), v = ldexp4(x[2 * m + 1], eq);
+        split_f16(f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w}, qh[m], ql[m]);
+      }
+      clip_kv(0, k0, v0);
+      clip_kv(last < 1 ? last : 1, ka, va);
+      note_max(k0, v0, 0);
+      note_max(ka, va, 1);
+      if (lane == 0) red[2][w][0] = red[2][w][1] = mq;
+      __syncthreads();
+      float mk, mv, q0, q1;
+      read_max(0, mk, mv);
+      read_max(2, q0, q1);
+      if (!(mk < INFINITY && mv < INFINITY && q0 < INFINITY)) {  // uniform; NaN too
+        wait_vmcnt<0>();  // no copy in flight when the LDS is released
+        return false;
+      }
+      ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
+      ev = value_exp(mv);
+      put(0, k0, v0, ek, ev);
+      __syncthreads();
+    }
+
+    f32x16 o = {};
+    float l_run = 0.f;
+    bool bad = false;  // a non-finite tile; uniform
+    auto run = [&](auto exact_tag) {
+      constexpr bool kExact = decltype(exact_tag)::value;
+      const f32x16 zero16 = {};
+      // Reference state of this lane's query: m_ref the largest tile max seen
+      // when the reference was last looked at (-inf: none yet).
+      float m_ref = -INFINITY;
+      float c_ref = 0.f;
+      float w_ref = 1.f;     // exact path: 2^-(m_ref log2(e) - c_ref)
+      bool has_ref = false;  // uniform per wave, as big
+      bool big = false;
+      // Logits x in natural units -> the weights' planes.
+      auto softmax = [&](const f32x16& x, bf16x8 (&ph)[2], bf16x8 (&pl)[2]) {
+        f32x16 p;
+        if (kExact) {
+          const float mt = xor32_max(max16(x));
+          if (__any(mt > m_ref + kRescaleNat)) {
+            const float m_new = __builtin_elementwise_maximum(m_ref, mt);
+            const float c_new = m_new == -INFINITY ? 0.f : m_new * kLog2e;
+            const float alpha = m_ref == -INFINITY ? 0.f : exp2_fast((m_ref - m_new) * kLog2e);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[r] *= alpha;
+            l_run *= alpha;
+            m_ref = m_new;
+            c_ref = c_new;
+            w_ref = m_new == -INFINITY ? 1.f : exp2_fast(-__builtin_fmaf(m_new, kLog2e, -c_new));
+          }
+          // P = p w_ref is at most 2^8; the planes hold P 2^kShift, the sum P 2^kShift too
+          const float f = w_ref * 128.0f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) p[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref)) * f;
+          l_run += sum16(p);
+        } else {
+          // Logits past 2^22 (big) are rounded to log2 units before the
+          // reference is taken off, so that none exceeds its own maximum.
+          auto weights = [&]() {
+            if (big) {
+#pragma clang fp contract(off)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) {
+                const float y = x[r] * kLog2e;
+                p[r] = exp2_fast(y - c_ref);
+              }
+            } else {
+#pragma unroll
+              for (int r = 0; r < 16; ++r) p[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref));
+            }
+          };
+          weights();
+          float ps = sum16(p);
+          if (!has_ref || __any(!(ps <= kPlaneMax))) {
+            // Rare, taken by the whole wavefront: the first tile, or a tile
+            // whose weights would leave the fp16 range.  The reference moves
+            // up to kShift below the tile's max rounded up to an integer; the
+            // previous sums scale by the exact power of two alpha.  A query
+            // whose logits are all -inf so far keeps no reference.
+            const float mt = xor32_max(max16(x)) * kLog2e;
+            const bool fresh = m_ref == -INFINITY;
+            m_ref = __builtin_elementwise_maximum(m_ref, mt);
+            const float top = __builtin_ceilf(mt);
+            const float to = __builtin_fabsf(top) < kBigLogit ? top - kShift : top;
+            const float c_new = fresh ? (m_ref == -INFINITY ? 0.f : to)
+                                      : __builtin_elementwise_maximum(c_ref, to);
+            const float alpha = fresh ? 0.f : exp2_fast(c_ref - c_new);  // 1 when unchanged
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[r] *= alpha;
+            l_run *= alpha;
+            c_ref = c_new;
+            has_ref = __all(m_ref != -INFINITY);
+            big = __any(!(__builtin_fabsf(c_ref) < kBigLogit));
+            weights();
+            ps = sum16(p);
+          }
+          l_run += ps;
+        }
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const f32x8 v = {p[8 * m + 0], p[8 * m + 1], p[8 * m + 2], p[8 * m + 3],
+                           p[8 * m + 4], p[8 * m + 5], p[8 * m + 6], p[8 * m + 7]};
+          split_f16(v, ph[m], pl[m]);
+        }
+      };
+
+      for (int t = 0; t <= last; ++t) {
+        const int par = t & 1;
+        const int e = eq + ek;  // of tile t
+        // Tile t + 1 into the other stage, which every wave left behind at the
+        // last barrier; then tile t + 2's rows on their way (clamped to the
+        // last tile).
+        int e_new = ev;
+        if (t < last) {
+          float mk, mv;
+          read_max(par ^ 1, mk, mv);
+          if (!(mk < INFINITY && mv < INFINITY)) {  // uniform; NaN too
+            bad = true;
+            break;
+          }
+          ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
+          e_new = min(ev, value_exp(mv));
+          put(par ^ 1, ka, va, ek, e_new);
+        }
+        load_kv(t + 2 <= last ? t + 2 : last, ka, va);
+        asm volatile("" ::: "memory");  // issued here: the wait below counts them
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 acc = zero16;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const bf16x8 kh = plane_rd(par, 0, m);
+          const bf16x8 kl = plane_rd(par, 1, m);
+          acc = mfma_f16(kl, qh[m], acc);
+          acc = mfma_f16(kh, ql[m], acc);
+          acc = mfma_f16(kh, qh[m], acc);
+        }
+        // The wave's bias fragment has landed once at most the five row loads
+        // above, issued after it, are outstanding.  When nothing reads those
+        // rows the compiler may drop the loads: wait for all.
+        if (t + 2 <= last)
+          wait_vmcnt<5>();
+        else
+          wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        f32x16 x = bias_rd();
+        const float st = __builtin_ldexpf(1.0f, -min(max(e, -126), 126));
+        if (kExact) {
+          with_mask(t, [&](int r, float m) { x[r] = ((acc[r] * st) + m) + x[r]; });
         } else {
 #pragma unroll
-          for (int r = 0; r < 16; ++r) p[r] = exp2_fast(x[r] - c_ref);
+          for (int r = 0; r < 16; ++r) x[r] = __builtin_fmaf(acc[r], st, x[r]);
+          if (masked(t)) with_mask(t, [&](int r, float m) { x[r] += m; });
         }
-        const float l_new = l_run + sum16(p);
-        const bool over = !(l_new <= kSumLimit);  // NaN or inf count as overflow
-        if (!__any(over)) {
-          l_run = l_new;
-          return;
+        bf16x8 ph[2], pl[2];
+        softmax(x, ph, pl);
+        if (t + 2 <= last) {
+          clip_kv(t + 2, ka, va);
+          note_max(ka, va, par);  // read in iteration t + 1
         }
-        ovf = over ? 1.f : 0.f;
-      }
-      // Rare path, taken by the whole wavefront.  A lane moves its reference
-      // only when it has none yet, when its own running sum overflowed, or
-      // when this tile's max lies more than kSnap above the reference; the
-      // decision is shared by the lane pair (l, l ^ 32) that holds the query.
-      // After a sum overflow the true row max is at least c_ref + 52, so the
-      // reference moves up by at least kLift and the weights stay below 2^24.
-      const float mt = xor32_max(max16(x));
-      const bool fresh = m_ref == -INFINITY;
-      const bool need = fresh || xor32_max(ovf) > 0.f || mt > c_ref + kSnap;
-      m_ref = __builtin_elementwise_maximum(m_ref, mt);
-      const float snapped =
-          (m_ref == -INFINITY || (m_ref >= -kSnap && m_ref <= kSnap)) ? 0.f : m_ref;
-      const float c_new = fresh ? snapped
-                          : need ? __builtin_elementwise_maximum(snapped, c_ref + kLift)
-                                 : c_ref;
-      const float alpha = fresh ? 0.f : exp2_fast(c_ref - c_new);  // 1 when unchanged
+        if (t < last) bias_dma(t + 1);  // the fragment's reads are done (softmax used them)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[r] *= alpha;
-      l_run *= alpha;
-      c_ref = c_new;
+        for (int m = 0; m < 2; ++m) {
+          const bf16x8 vh = plane_rd(par, 2, m);
+          const bf16x8 vl = plane_rd(par, 3, m);
+          o = mfma_f16(vl, ph[m], o);
+          o = mfma_f16(vh, pl[m], o);
+          o = mfma_f16(vh, ph[m], o);
+        }
+        if (t < last) {
+          if (e_new != ev) {  // uniform: O to the scale of tile t + 1
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = exp2_fast(x[r] - c_ref);
-      l_run += sum16(p);
-      has_ref = __all(m_ref != -INFINITY);
-      c_zero = __all(c_ref == 0.f);
-    };
-
-    auto bias_of = [&](int t) -> f32x16 { return kExact ? io.bias(t) : io.bias_l2(t); };
-
-    // Prologue: K(0), V(0) into LDS; K(1), V(1) and the biases of tiles 0
-    // and 1 in flight.
-    f32x16 set_a = bias_of(0);
-    f32x16 set_b = bias_of(last < 1 ? last : 1);
-    {
-      const f32x4 k0 = io.k(0);
-      const f32x4 v0 = io.v(0);
-      *(f32x4*)&Ks[0][row8][col4] = k0;
-      Tiles<LAYOUT>::store_v(Vs[0], v0, row8, col4);
-    }
-    f32x4 kreg = io.k(last < 1 ? last : 1);
-    f32x4 vreg = io.v(last < 1 ? last : 1);
-    __syncthreads();
-
-    // Tile kt: Ks/Vs[kt&1] hold K(kt), V(kt); x holds bias(kt); kreg/vreg
-    // hold K(kt+1), V(kt+1) (loads in flight).  Indices past the last tile
-    // are clamped (in range, never used).
-    auto body = [&](int kt, f32x16& x) {
-      const int par = kt & 1;
-      if (kExact) {
-        p = qk_chain(Ks[par], qf, l32, half, zero16);
-        const f32x16 mb = mask_vals(kt);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = (p[r] + mb[r]) + x[r];
-      } else {
-        // The dot product accumulates from zero (its partial sums round at
-        // its own magnitude, not at the bias's), then one fma adds the
-        // log2(e)-scaled bias: log2-domain logits at FP32 accuracy.
-        p = qk_chain(Ks[par], qf, l32, half, zero16);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = __builtin_fmaf(p[r], kLog2e, x[r]);
-        if (masked(kt)) {
-          const f32x16 mb = mask_vals(kt);
-#pragma unroll
-          for (int r = 0; r < 16; ++r) x[r] = __builtin_fmaf(mb[r], kLog2e, x[r]);
+            for (int r = 0; r < 16; ++r) o[r] = __builtin_ldexpf(o[r], e_new - ev);
+            ev = e_new;
+          }
+          __syncthreads();
         }
       }
-      softmax(x);
-      x = bias_of(kt + 2 < last ? kt + 2 : last);
-      pv(Vs[par], p);
-      *(f32x4*)&Ks[par ^ 1][row8][col4] = kreg;
-      Tiles<LAYOUT>::store_v(Vs[par ^ 1], vreg, row8, col4);
-      kreg = io.k(kt + 2 < last ? kt + 2 : last);
-      vreg = io.v(kt + 2 < last ? kt + 2 : last);
-      __syncthreads();
     };
-
-    int kt = 0;
-    for (; kt + 1 < nkt; kt += 2) {
-      body(kt, set_a);
-      body(kt + 1, set_b);
+    if (has_unmasked) {
+      run(std::false_type{});
+    } else {
+      run(std::true_type{});
     }
-    if (kt < nkt) body(kt, set_a);
+    wait_vmcnt<0>();  // no copy in flight when the LDS is released
+    if (bad) return false;
+
+    const float l_tot = xor32_sum(l_run);
+    if (jq < a.n) {
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int c = 8 * rr + 4 * half;  // channels c..c+3 of head h
+        f32x4 ov = {__builtin_ldexpf(o[4 * rr + 0], -ev) / l_tot,
+                    __builtin_ldexpf(o[4 * rr + 1], -ev) / l_tot,
+                    __builtin_ldexpf(o[4 * rr + 2], -ev) / l_tot,
+                    __builtin_ldexpf(o[4 * rr + 3], -ev) / l_tot};
+        *(f32x4*)(a.out + (((int64_t)b * a.n + jq) * kHeads + h) * kHeadDim + c) = ov;
+      }
+    }
+    return true;
   };
-  if (has_unmasked) {
-    run(std::false_type{});
-  } else {
-    run(std::true_type{});
-  }
-
-  const float l_tot = xor32_sum(l_run);
-  if (jq < a.n) {
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      const int c = 8 * rr + 4 * half;  // channels c..c+3 of head h
-      f32x4 ov = {o[4 * rr + 0] / l_tot, o[4 * rr + 1] / l_tot, o[4 * rr + 2] / l_tot,
-                  o[4 * rr + 3] / l_tot};
-      *(f32x4*)(a.out + (((int64_t)b * a.n + jq) * kHeads + h) * kHeadDim + c) = ov;
-    }
-  }
+  if (!attend()) attend_scalar(a, b, h, jq, half);
 }
 
 }  // namespace
@@ -397,8 +497,9 @@ hipError_t launch_attention(int layout, const AttnArgs& a, hipStream_t stream) {
   const uint64_t total = groups * kRowGroup * kHeads * nqt;
   if (total == 0) return hipSuccess;
   if (total > 0x7fffffffull) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(attention_kernel<kAttnHeadLast>, dim3((uint32_t)total), dim3(kThreads), 0,
-                     stream, a, nqt, nkt, (uint32_t)total);
+  const int ppg = pair_group_size(nqt, (uint64_t)kBq * (uint64_t)a.n * sizeof(float));
+  hipLaunchKernelGGL(attention_kernel, dim3((uint32_t)total), dim3(kThreads), 0, stream, a, nqt,
+                     nkt, (uint32_t)total, ppg);
   return hipGetLastError();
 }
 

@@ -99,14 +99,15 @@ __device__ __forceinline__ int v_position(int g) {
 // (padding rows: inf (mask - 1) = -1e9), when the products are bounded below
 // half the float32 spacing next to m on either side: then fl(s + m) = m for
 // every key (|s| <= max|q|_2 max|k|_2 over the row's queries and keys, with a
-// margin for the native rounding of s), so the native logit fl(fl(s + m) + bias) is fl(m + bias), the same
-// for every such row.  With |m| = f 2^e, f in [0.5, 1), the spacing above
-// |m| is 2^(e - 24); toward zero it is the same unless |m| is a power of two
-// (f = 0.5), where it halves.  The row's own 2-norms bound s about 7 times
-// closer than 32 max|q| max|k| over the whole pair would (unit-scale q and k
-// at N = 1536: 16 against 114, the limit at m = -1e9 being 32), which keeps
-// ordinary padding rows off the exact softmax: 184 rows of 1536 take 0.3 ms
-// with their shared weights against 1.10 ms there.
+// margin for the native rounding of s), so the native logit fl(fl(s + m) +
+// bias) is fl(m + bias), the same for every such row.  With |m| = f 2^e, f in
+// [0.5, 1), the spacing above |m| is 2^(e - 24); toward zero it is the same
+// unless |m| is a power of two (f = 0.5), where it halves.  The row's own
+// 2-norms bound s about 7 times closer than 32 max|q| max|k| over the whole
+// pair would (unit-scale q and k at N = 1536: 16 against 114, the limit at
+// m = -1e9 being 32), which keeps ordinary padding rows off the exact softmax:
+// 184 rows of 1536 take 0.3 ms with their shared weights against 1.10 ms
+// there.
 __device__ __forceinline__ bool constant_mask_row(const AttnArgs& a, int b, float& m) {
   if (a.magnitudes == nullptr || a.magnitudes[4] != 1u) return false;
   if (!constant_mask(a.tile_flags, b, m)) return false;

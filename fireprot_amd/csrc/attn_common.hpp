@@ -1,5 +1,5 @@
-// Helpers shared by the FP32-accurate attention kernels (attention.hip on the
-// FP32 matrix cores, attention_split.hip on the 16-bit matrix cores, bf16.hip): buffer
+// Helpers shared by the attention kernels (attention.hip, attention_split.hip,
+// bf16.hip): buffer
 // loads, the lane-pair exchanges of the transposed S^T / O^T layout, row
 // reductions, and the softmax reference constants.
 #pragma once

@@ -1,8 +1,8 @@
 // Shared device helpers for the gfx950 triangle-attention kernels.
 //
-// Everything here is CDNA4-specific: 64-lane wavefronts, the FP32 matrix-core
-// instruction v_mfma_f32_32x32x2_f32, and an XCD-aware work-group remap for the
-// 8 accelerator dies of an MI355X.
+// Everything here is CDNA4-specific: 64-lane wavefronts, the matrix cores'
+// result layout, and an XCD-aware work-group remap for the 8 accelerator dies
+// of an MI355X.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,17 +23,9 @@ constexpr int kHidden = kHeads * kHeadDim;  // 128
 constexpr int kXcds = 8;
 constexpr float kLog2e = 1.4426950408889634f;
 
-// D = A x B + C for one 32x32x2 FP32 matrix-core step.
-// Operand/result lane layouts (CDNA3/CDNA4 ISA, "32x32x2 f32", single block):
-//   A[row][k]  : lane = row + 32*k                      (row 0..31, k 0..1)
-//   B[k][col]  : lane = col + 32*k
-//   D[row][col]: lane = col + 32*((row/4)%2), register = (row%4) + 4*(row/8)
-// i.e. lane l, register r holds D[8*(r/4) + 4*(l/32) + r%4][l%32].
-// tests/test_gpu_mfma_layout.py calibrates this on the device.
-__device__ __forceinline__ f32x16 mfma32(float a, float b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
+// FP32 result layout of the 32x32 matrix-core instructions (32x32x16 f16 and
+// bf16 here): D[row][col] in lane col + 32*((row/4)%2), register (row%4) +
+// 4*(row/8), i.e. lane l, register r holds D[8*(r/4) + 4*(l/32) + r%4][l%32].
 // Row index (0..31) of result register r in lane half `half` (= lane/32).
 __device__ __forceinline__ int mfma_row(int r, int half) {
   return 8 * (r >> 2) + 4 * half + (r & 3);
@@ -131,22 +123,6 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t total) {
   const uint32_t slot = b / kXcds;
   return xcd < extra ? xcd * (per + 1) + slot
                      : extra * (per + 1) + (xcd - extra) * per + slot;
-}
-
-// [128 x 32] weight fragment (B operand of v_mfma_f32_32x32x2_f32) of output
-// column col (this lane's l % 32) of a torch [out][in] weight with in
-// stride ld: lane half h holds input channels 64h .. 64h + 63.
-__device__ __forceinline__ void load_fragment(const float* w, int col, int half, float* wf,
-                                              int64_t ld = kChannels) {
-  const float* src = w + (int64_t)col * ld + 64 * half;
-#pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    const f32x4 v = *(const f32x4*)(src + 4 * t);
-    wf[4 * t + 0] = v.x;
-    wf[4 * t + 1] = v.y;
-    wf[4 * t + 2] = v.z;
-    wf[4 * t + 3] = v.w;
-  }
 }
 
 __host__ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) {

@@ -131,10 +131,9 @@ struct AttnArgs {
   int np;
 };
 
-// launch_attention: kAttnHeadLast (the reference C-ABI layout) on the FP32
-// matrix cores (attention_kernel).  launch_attention_split runs
-// attention_split_kernel (FP32-accurate products on the 16-bit matrix cores)
-// for kAttnBlock or kAttnStaged.
+// launch_attention: kAttnHeadLast (the reference C-ABI layout), operands split
+// into planes in the kernel (attention_kernel).  launch_attention_split runs
+// attention_split_kernel on staged planes for kAttnBlock or kAttnStaged.
 hipError_t launch_attention(int layout, const AttnArgs& args, hipStream_t stream);
 hipError_t launch_attention_split(int layout, const AttnArgs& args, hipStream_t stream);
 // The FP32 block after its projection: rewrite bias_l2 ([4][np][np],

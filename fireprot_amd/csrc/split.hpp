@@ -11,7 +11,7 @@
 //
 // Operand lane layout of v_mfma_f32_32x32x16_{f16,bf16} (one block): lane l
 // holds A[l % 32][8 * (l / 32) + e] and B[8 * (l / 32) + e][l % 32],
-// e = 0..7, of one 16-deep k step; the FP32 result has the 32x32x2 f32 layout
+// e = 0..7, of one 16-deep k step; the FP32 result has the 32x32 layout
 // (common.hpp).
 #pragma once
 

@@ -1,0 +1,104 @@
+"""``fpx_attn_core_masked`` splits its operands into fp16 planes tile by tile:
+the cases where a plane exponent, a softmax reference or the plane form itself
+has to give way, against plain torch in float64.
+
+Bar: the largest error within max(2e-6 of the largest value, twice the error of
+the same expression in FP32 torch); NaN and infinities where torch has them.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fireprot_amd import _native
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(batch, n, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q, k, v = (torch.randn(batch, n, 4, 32, device="cuda", generator=g) for _ in range(3))
+    return q / 32 ** 0.5, k, v, torch.randn(4, n, n, device="cuda", generator=g)
+
+
+def _run(q, k, v, bias, mask=None, row=None):
+    batch, n = q.shape[:2]
+    out = torch.full_like(q, 7.0)
+    _native.check(_native.library().fpx_attn_core_masked(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), None if mask is None else mask.data_ptr(),
+        0 if mask is None else n, bias.data_ptr(), row or n, out.data_ptr(), batch, n,
+        torch.cuda.current_stream().cuda_stream), "fpx_attn_core_masked")
+    return out
+
+
+def _torch(q, k, v, bias, mask, dtype):
+    q, k, v = (t.to(dtype).permute(0, 2, 1, 3).contiguous() for t in (q, k, v))
+    s = torch.matmul(q, k.transpose(2, 3).contiguous())
+    if mask is not None:
+        s = s + mask.to(dtype)[:, None, None, :]
+    return torch.matmul(torch.softmax(s + bias.to(dtype), -1), v).permute(0, 2, 1, 3)
+
+
+def _check(q, k, v, bias, mask=None):
+    out = _run(q, k, v, bias, mask).double()
+    ref = _torch(q, k, v, bias, mask, torch.float64)
+    low = _torch(q, k, v, bias, mask, torch.float32).double()
+    bar = max(2e-6 * ref.abs().max().item(), 2.0 * (low - ref).abs().max().item())
+    err = (out - ref).abs().max().item()
+    assert err <= bar, (err, bar)
+
+
+@pytest.mark.parametrize("n", [4, 28, 32, 36, 64, 100, 128, 132, 260])
+@pytest.mark.parametrize("masked", [False, True])
+def test_tile_edges(n, masked):
+    q, k, v, bias = _inputs(3, n, n)
+    mask = None
+    if masked:
+        mask = 1e9 * ((torch.arange(n, device="cuda") % 3 != 1).float() - 1.0).repeat(3, 1)
+    _check(q, k, v, bias, mask)
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("scales", [(1e-6, 1.0, 1e4), (1e4, 1.0, 1e-6), (0.0, 1.0, 0.0),
+                                    (1e-30, 1e-33, 1e-36)])
+def test_tiles_of_different_magnitudes(which, scales):
+    """Each 32-key tile at its own scale: V's exponent falls (O is rescaled)
+    and rises, a zero tile sets none, values far below the others stay."""
+    n = 160
+    q, k, v, bias = _inputs(2, n, 5)
+    s = torch.tensor(scales, device="cuda")[(torch.arange(n, device="cuda") // 32) % 3]
+    t = {"q": q, "k": k, "v": v}[which]
+    t.mul_(s[None, :, None, None] if which != "k" else s[None, :, None, None].clamp(max=30.0))
+    _check(q, k, v, bias)
+
+
+@pytest.mark.parametrize("gain", [30.0, 1e4, 3e7, 1e9])
+def test_wide_logits_move_the_reference(gain):
+    """Logits that rise from tile to tile, past 2^22 in log2 units too."""
+    n = 132
+    q, k, v, bias = _inputs(2, n, 9)
+    bias = bias * gain + gain * torch.arange(n, device="cuda") / 16.0
+    _check(q, k, v, bias)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("which", ["q", "k", "v", "bias"])
+@pytest.mark.parametrize("key", [3, 70, 99])
+def test_non_finite_inputs_as_torch(which, value, key):
+    n = 100
+    q, k, v, bias = _inputs(2, n, 11)
+    if which == "bias":
+        bias[1, 5, key] = value
+    else:
+        {"q": q, "k": k, "v": v}[which][0, key, 2, 7] = value
+    out, ref = _run(q, k, v, bias), _torch(q, k, v, bias, None, torch.float32)
+    torch.testing.assert_close(out, ref, atol=2e-5, rtol=2e-5, equal_nan=True)
+
+
+def test_bias_rows_beyond_32_bit_offsets():
+    n, row = 4, (1 << 25) + 4
+    q, k, v, bias = _inputs(2, n, 13)
+    rows = torch.empty(4 * n, row, device="cuda")
+    rows[:, :n] = bias.view(4 * n, n)
+    out = _run(q, k, v, rows, row=row)
+    torch.testing.assert_close(out, _torch(q, k, v, bias, None, torch.float32), atol=2e-6, rtol=0)
