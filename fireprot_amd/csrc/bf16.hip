@@ -57,7 +57,12 @@ __global__ __launch_bounds__(Bf16ProjTraits<MODE>::kWaves * 64) void projection_
   constexpr int NW = Bf16ProjTraits<MODE>::kWaves;
   constexpr bool kLn = Bf16ProjTraits<MODE>::kLn;
   constexpr int kThreads = NW * 64;
-  constexpr int kRowsPerWave = kRows / NW;
+  // LN mode: two rows per wave, 32 lanes per row, lane l32 holding channels
+  // 4 l32 .. + 3 of row 2 w + half: one pass of half-wave reductions serves
+  // both rows, and the four bias heads share one (half_sum4).  With a row per
+  // wave pass and a 64-lane reduction per statistic and head, the VALU work
+  // held the launch at small N: 69 us at N = 384, now 59.
+  static_assert(!kLn || 2 * NW == kRows, "two rows per wave");
   constexpr int kVecs = kRows * kChannels / 8;               // 16-byte vectors per tile
   constexpr int kLoads = (kVecs + kThreads - 1) / kThreads;
   // Two row tiles: the MFMAs read one while the next is normalised into the
@@ -80,30 +85,20 @@ __global__ __launch_bounds__(Bf16ProjTraits<MODE>::kWaves * 64) void projection_
   const int col_w = MODE == kProjOut ? 32 * w + l32 : 32 * (w & 3) + l32;
   const float col_bias = a.bias_vec != nullptr ? (float)a.bias_vec[col_w] : 0.f;
 
-  float lnw[2] = {1.f, 1.f}, lnb[2] = {0.f, 0.f};
-  float wb[kHeads][2] = {};
-  if (kLn) {
-    if (a.ln_w) {
-      const bf16x2 v = *(const bf16x2*)(a.ln_w + 2 * lane);
-      lnw[0] = (float)v.x;
-      lnw[1] = (float)v.y;
-    }
-    if (a.ln_b) {
-      const bf16x2 v = *(const bf16x2*)(a.ln_b + 2 * lane);
-      lnb[0] = (float)v.x;
-      lnb[1] = (float)v.y;
-    }
+  __shared__ __attribute__((aligned(16))) float wbias[kLn ? kHeads : 1][kLn ? kChannels : 4];
+  f32x4 lnw = {1.f, 1.f, 1.f, 1.f}, lnb = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (kLn) {
 #pragma unroll
-    for (int h = 0; h < kHeads; ++h) {
-      const bf16x2 v = *(const bf16x2*)(a.w_bias + h * kChannels + 2 * lane);
-      wb[h][0] = (float)v.x;
-      wb[h][1] = (float)v.y;
+    for (int e = 0; e < 4; ++e) {
+      if (a.ln_w) lnw[e] = (float)a.ln_w[4 * l32 + e];
+      if (a.ln_b) lnb[e] = (float)a.ln_b[4 * l32 + e];
     }
+    if (tid < kHeads * kChannels) wbias[tid >> 7][tid & 127] = (float)a.w_bias[tid];
+    __syncthreads();
   }
 
-  bf16x2 stage_ln[kLn ? kRowsPerWave : 1];
+  bf16x4 stage_ln = {};
   bf16x8 stage_vec[kLn ? 1 : kLoads];
-  const bf16x2 zero2 = {(__bf16)0.f, (__bf16)0.f};
   const bf16x8 zero8 = {(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f,
                         (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
 
@@ -111,13 +106,9 @@ __global__ __launch_bounds__(Bf16ProjTraits<MODE>::kWaves * 64) void projection_
     const int i = tile / tiles_j;
     const int j0 = (tile % tiles_j) * kRows;
     if (kLn) {
-#pragma unroll
-      for (int rr = 0; rr < kRowsPerWave; ++rr) {
-        const int j = j0 + w * kRowsPerWave + rr;
-        stage_ln[rr] = j < a.rows_j
-                           ? *(const bf16x2*)(a.x + (int64_t)i * a.xs_i + (int64_t)j * a.xs_j + 2 * lane)
-                           : zero2;
-      }
+      // a row past the last is read from it and zeroed by stage_rows
+      const int j = min(j0 + 2 * w + half, a.rows_j - 1);
+      stage_ln = *(const bf16x4*)(a.x + (int64_t)i * a.xs_i + (int64_t)j * a.xs_j + 4 * l32);
     } else {
 #pragma unroll
       for (int t = 0; t < kLoads; ++t) {
@@ -137,29 +128,34 @@ __global__ __launch_bounds__(Bf16ProjTraits<MODE>::kWaves * 64) void projection_
     const int i = tile / tiles_j;
     const int j0 = (tile % tiles_j) * kRows;
     if (kLn) {
+      const int row = 2 * w + half;
+      const int j = j0 + row;
+      const bool valid = j < a.rows_j;
+      // Two-pass statistics of the values shifted by the row's first channel
+      // (as ln_stats_c128).
+      f32x4 x = {(float)stage_ln.x, (float)stage_ln.y, (float)stage_ln.z, (float)stage_ln.w};
+      const int first = __builtin_bit_cast(int, (float)stage_ln.x);
+      const float pivot = __builtin_bit_cast(
+          float, half ? __builtin_amdgcn_readlane(first, 32) : __builtin_amdgcn_readlane(first, 0));
+      x = x - pivot;
+      x = x - half_sum((x.x + x.y) + (x.z + x.w)) * (1.0f / kChannels);
+      const float var =
+          half_sum((x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w)) * (1.0f / kChannels);
+      f32x4 y = x * __builtin_amdgcn_rsqf(var + a.eps) * lnw + lnb;
+      if (!valid) y = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bf16x4 yb = {(__bf16)y.x, (__bf16)y.y, (__bf16)y.z, (__bf16)y.w};
+      *(bf16x4*)&xs[buf][row][4 * l32] = yb;
+      if constexpr (MODE == kProjBlock) {
+        const f32x4 r = {(float)yb.x, (float)yb.y, (float)yb.z, (float)yb.w};
+        float p[kHeads];
 #pragma unroll
-      for (int rr = 0; rr < kRowsPerWave; ++rr) {
-        const int row = w * kRowsPerWave + rr;
-        const int j = j0 + row;
-        const bool valid = j < a.rows_j;
-        float d0, d1, rstd;
-        ln_stats_c128((float)stage_ln[rr].x, (float)stage_ln[rr].y, a.eps, d0, d1, rstd);
-        float y0 = d0 * rstd * lnw[0] + lnb[0];
-        float y1 = d1 * rstd * lnw[1] + lnb[1];
-        if (!valid) y0 = y1 = 0.f;
-        const bf16x2 yb = {(__bf16)y0, (__bf16)y1};
-        *(bf16x2*)&xs[buf][row][2 * lane] = yb;
-        if (MODE == kProjBlock) {
-          const float r0 = (float)yb.x;
-          const float r1 = (float)yb.y;
-          float p[kHeads];
-#pragma unroll
-          for (int h = 0; h < kHeads; ++h) p[h] = wave_sum(r0 * wb[h][0] + r1 * wb[h][1]);
-          if (lane < kHeads) {
-            const float v = lane == 0 ? p[0] : lane == 1 ? p[1] : lane == 2 ? p[2] : p[3];
-            a.tri_bias[bias_frag_index_bf16(lane, i, j, a.np)] = (__bf16)(valid ? v * kLog2e : 0.f);
-          }
+        for (int h = 0; h < kHeads; ++h) {
+          const f32x4 wb = *(const f32x4*)&wbias[h][4 * l32];
+          p[h] = (r.x * wb.x + r.y * wb.y) + (r.z * wb.z + r.w * wb.w);
         }
+        const float v = half_sum4(p[0], p[1], p[2], p[3], lane);
+        if (l32 < kHeads)
+          a.tri_bias[bias_frag_index_bf16(l32, i, j, a.np)] = (__bf16)(valid ? v * kLog2e : 0.f);
       }
     } else {
 #pragma unroll
@@ -269,17 +265,19 @@ __global__ __launch_bounds__(Bf16ProjTraits<MODE>::kWaves * 64) void projection_
   int next = tile + (int)gridDim.x;
   if (next < ntiles) fetch(next);
   __syncthreads();
-  // A tile's results are stored one iteration late, right after the next
-  // tile's rows are staged: loads and stores share one counter, and the
-  // wait for the staged rows' loads then finds the stores a full iteration
-  // old instead of waiting for their completion.
+  // A tile's results are stored one iteration late, after the next tile's
+  // rows are staged and the loads of the tile after it are issued: loads and
+  // stores share one counter, and the wait for a tile's rows then finds only
+  // stores a full iteration old before its loads.  (Loads issued after the
+  // stores: 9.66 ms per ending-node block at N = 2048, before them 9.38;
+  // loads a further tile ahead in a second register slot: 9.60.)
   f32x16 acc_prev = {};
   int prev_tile = -1;
   for (int buf = 0; tile < ntiles; buf ^= 1) {
     const f32x16 acc = mfma_tile(buf);
     if (next < ntiles) stage_rows(next, buf ^ 1);
-    if (prev_tile >= 0) epilogue(prev_tile, acc_prev);
     if (next < ntiles && next + (int)gridDim.x < ntiles) fetch(next + gridDim.x);
+    if (prev_tile >= 0) epilogue(prev_tile, acc_prev);
     acc_prev = acc;
     prev_tile = tile;
     __syncthreads();

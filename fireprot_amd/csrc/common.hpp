@@ -84,6 +84,33 @@ __device__ __forceinline__ float half_max(float v) {
   return mx(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
 }
 
+// Sum over each 32-lane half of the wave, returned in every lane of the half.
+__device__ __forceinline__ float half_sum(float v) {
+  v += dpp<0xB1>(v);
+  v += dpp<0x4E>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
+// Sums of four values over each 32-lane half: lane l returns that of value
+// l % 4.  Lane pairs and then quads each keep one value (three instructions per
+// pair instead of a full reduction per value), which row_ror:4 and :8 and the
+// row exchange then sum: 14 instructions for the four.
+__device__ __forceinline__ float half_sum4(float p0, float p1, float p2, float p3, int lane) {
+  const bool odd = lane & 1, upper = lane & 2;
+  const float a = (odd ? p1 : p0) + dpp<0xB1>(odd ? p0 : p1);
+  const float b = (odd ? p3 : p2) + dpp<0xB1>(odd ? p2 : p3);
+  float v = (upper ? b : a) + dpp<0x4E>(upper ? a : b);
+  v += dpp<0x124>(v);
+  v += dpp<0x128>(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+
 // Two-pass LayerNorm statistics of a 128-channel row held as two values per
 // lane.  Values are shifted by lane 0's first value before summing, so rows
 // with |mean| >> std (e.g. 1000 + 0.001*c) keep their digits: the centred
