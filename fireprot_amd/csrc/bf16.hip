@@ -456,8 +456,9 @@ __global__ __launch_bounds__(kThreads, 3) void attention_bf16_kernel(Bf16AttnArg
   };
 
   // Q, the B operand of S^T: lane holds Q[jq][16m + 8half + e].
-  bf16x8 qf[2];
-  {
+  // Queries past the tile that holds n - 1 have no q: they run as zeros.
+  bf16x8 qf[2] = {};
+  if (j0 + 32 * w < a.n) {  // uniform per wave
     const __bf16* src = a.q + (bh * a.np + jq) * kHeadDim + 8 * half;
     qf[0] = *(const bf16x8*)(src);
     qf[1] = *(const bf16x8*)(src + 16);

@@ -410,7 +410,7 @@ int fpx_tri_attn_prepare(int dtype, const void* z, int64_t z_stride0, int64_t z_
     p.xs_j = xs_j;
     p.rows_i = n;
     p.rows_j = n;
-    p.span_j = w.np;
+    p.span_j = (int)round_up(n, 32);  // as the FP32 block's, below
     p.ln_w = static_cast<const __bf16*>(ln_w);
     p.ln_b = static_cast<const __bf16*>(ln_b);
     p.eps = eps;
