@@ -1255,7 +1255,7 @@ __device__ __forceinline__ void row_norms(const AttnArgs& a, uint32_t* tile_flag
 // minimised over the rows that have an unmasked key (so keys of tiles t < T
 // are unmasked on every row the fast softmax serves); nkt when no row has a
 // masked key.  C_q = ceil of query q's largest log2 bias over tiles t < T;
-// every tile of the query is then rewritten as bias_l2 - (C_q - kRelOffset),
+// every visited tile of the query is then rewritten as bias_l2 - (C_q - kRelOffset),
 // one rounding.  With T = 0 nothing is rewritten and the flag stays 0.
 //
 // Shared weights (kWeights: the call has a mask; else no row has a constant
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(kBiasWaves * 64) void pair_bias_kernel(AttnArgs a, 
     // values are never read, and keep the copy as it is
     const float c = __builtin_ceilf(over_waves(m));
     const float shift = __builtin_fabsf(c) < 4194304.0f ? c - kRelOffset : 0.0f;
-    for (int t = w; t < nt; t += kBiasWaves) {
+    for (int t = w; t < nkt; t += kBiasWaves) {
       float* dst = bias_l2 + frag + (int64_t)t * 1024;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {

@@ -15,7 +15,7 @@ triangle bias ``[1, 4, N, N]`` (any strides) and optionally the mask bias
 ``fpx_attn_strided`` (q, k, v staged into power-of-two scaled fp16 planes,
 then the block's attention kernel on the 16-bit matrix cores, FP32-accurate)
 with a workspace cached per device and stream; the reference's workspace-less
-entries ``ck_attention*`` stay on the FP32 matrix cores.
+entries ``ck_attention*`` split their operands in the kernel.
 
 ``triangle_attention_block`` -- the whole module call ``(z, mask) -> dz``,
 as AtlasFold's per-instance hook dispatches it
