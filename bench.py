@@ -38,7 +38,6 @@ ROOT = pathlib.Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
 METRIC = "triangle-attn block ms + TFLOP/s (% MFMA peak) at N=1536 FP32, 1 GPU"
-FP32_MFMA_PEAK_TFLOPS = 157.3
 BF16_MFMA_PEAK_TFLOPS = 2500.0
 HBM_PEAK_GBPS = 8000.0
 TRAFFIC_FILE = ROOT / "profiles" / "attention_traffic.json"
@@ -737,7 +736,7 @@ def bench_core(args) -> dict:
       - ``ck_attention_exact1536`` / ``ck_attention_vector_bias1000``: the
         reference's C ABI entries called as its ``attention()`` calls them
         (ck_attention.py:115-141: the bias packed into 1552-float rows at
-        N=1536), on the FP32 matrix cores.
+        N=1536), operands split into fp16 planes in the kernel.
     ``value``: the dispatch route at B=512, N=1536.  Every record carries the
     FP32 bar on four batch rows against the float64 oracle.
     """
@@ -805,7 +804,7 @@ def bench_core(args) -> dict:
             # result is [B, N, 4, 32]; the oracle's layout is [B, 4, N, 32]
             parity = strict_rows(f"{name} b={batch} n={n}", result.transpose(1, 2), q, k, v,
                                  [bias], rows)
-            peak = BF16_MFMA_PEAK_TFLOPS if name == "dispatch" else FP32_MFMA_PEAK_TFLOPS
+            peak = BF16_MFMA_PEAK_TFLOPS  # fp16 planes on both routes
             rec = {"route": name, "batch": batch, "n": n, "median_ms": round(median, 4),
                    "p95_ms": round(p95(times), 4), "min_ms": round(min(times), 4),
                    "tflops": round(flop / (median * 1e-3) / 1e12, 3),
@@ -1202,7 +1201,7 @@ def main() -> int:
             flops["core"] / (stages["attend"] * 1e-3) / 1e12, 3),
     }
     if split:
-        # padding rows of a tail mask take the constant-mask kernel (no S^T)
+        # padding rows of a tail mask run on shared weights (no S^T)
         const_tiles = 0 if cfg.valid is None or cfg.valid >= n else (n - cfg.valid) * nkt
         roofline.update(split_executed(n, n, stages["attend"], visited,
                                        const_tiles=const_tiles))

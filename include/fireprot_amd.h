@@ -171,8 +171,9 @@ int fpx_attn_core(float* q, float* k, float* v, float* bias, float* out, int bat
  *                                (fireprot_ck_attention.cpp:102-107)
  * A null or misaligned (16-byte) pointer returns 3 before any launch, as the
  * reference's vector_bias1000 entry does (fireprot_ck_attention.cpp:106-107);
- * the computation is FP32 on the FP32 matrix cores (v_mfma_f32_32x32x2_f32),
- * asynchronous on the caller's stream, with no allocation. */
+ * the computation is FP32-accurate on the 16-bit matrix cores (operands split
+ * into power-of-two scaled fp16 planes in the kernel; plain FP32 where q, k or
+ * v is not finite), asynchronous on the caller's stream, with no allocation. */
 int ck_attention(float* q, float* k, float* v, float* bias, float* out, int batch, int n,
                  void* stream);
 int ck_attention_exact1536(float* q, float* k, float* v, float* bias, float* out, int batch,
