@@ -47,6 +47,33 @@
 // so a work-group that meets a non-finite q, k or v computes its rows in plain
 // FP32 (attend_scalar) with the native propagation.
 //
+// Range.  A plane pair resolves 2^-25 in scaled units, 2^-39 of the largest
+// value it is scaled with, whereas FP32 keeps 24 bits of every value.  A
+// work-group whose operands need more runs on the FP32 matrix cores
+// (attend_f32):
+//   - logits: what the planes drop of one logit is at most 32 products of one
+//     operand's largest value and the other's resolution, for both operands:
+//     64 2^-39 max|q| max|K| = 2^-33 max|q| max|K|.  Up to max|q| max|K| =
+//     2^10 (kMaxProduct) that is 2^-23, the rounding of a logit near 1.  Past
+//     it the planes stay when no nonzero row and no nonzero channel of the
+//     wave's q or of the tile's K lies below 2^-8 of the largest value
+//     (kEvenShare): then they drop at most 2^-39 sqrt(32) 2 2^8 |q|_2 |k|_2 =
+//     2^-27.5 |q|_2 |k|_2, less than FP32 sums round.
+//   - V, looked at when the sums are complete, in scaled units (max|V| in
+//     [2^14, 2^15)): what the planes drop of O' = sum P' V' is at most
+//     2^-25 l' (V's resolution) and about 2^-25 2^14 sqrt(N / 3) (that of the
+//     weights, uniformly distributed errors of random sign).  A query whose
+//     largest |O'| over the channels is not 2^22 times that sum (kRowShare,
+//     kWeightShare) gets its weight from keys of V far below the largest (a
+//     masked key's, say): FP32.  Likewise when some channel's largest |V| is
+//     nonzero and below 1, 2^-14 or less of all: its error would pass 2^-25
+//     of it.
+// Tiles of V further apart than 2^20 (kMaxSpread; padded keys holding anything
+// are the usual cause) go to FP32 as they are met.  So the planes' error is
+// relative to the largest output of the row and to the largest V of the
+// channel.  The looks cost 1.3% at N = 1536 (3118 to 3160 us) and at most
+// 0.6 us of 13 at N = 128.
+//
 // Bound: VALU issue beside the matrix cores (about 170 VALU instructions and
 // 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.23 ms; on the FP32
 // matrix cores, which never overlap with VALU work, 5.42 ms.  N = 384 175 us
@@ -70,6 +97,26 @@ constexpr float kPlaneMax = 32768.0f;          // bound on a lane's 16 scaled we
 constexpr float kShift = 7.0f;                 // weights enter P.V as up to 2^7 and more
 constexpr int64_t kMaxBiasStride = 1 << 25;    // 31 rows within 32-bit byte offsets
 constexpr float kBigLogit = 4194304.0f;        // 2^22: past it, references take no shift
+// Range of the planes (file comment); 2^22 times 2^-25 and 2^-25 2^14 / sqrt(3).
+constexpr float kMaxProduct = 1024.0f;
+constexpr float kEvenShare = 0x1p-8f;
+constexpr float kRowShare = 0.125f;
+constexpr float kWeightShare = 1182.4f;
+constexpr int kMaxSpread = 20;
+constexpr int kNoExp = 141;  // V's exponent while every tile was zero
+
+// The planes' ring and bias fragments; attend_f32's K and V tiles in their place.
+constexpr int kPad = 4;  // LDS row padding (floats): conflict-free b128 reads
+typedef float KTile[kBk][kHeadDim + kPad];  // [key][channel]
+typedef float VTile[kHeadDim][kBk + kPad];  // [channel][key]
+constexpr int kPoolBytes = 2 * kTileBytes + kThreads / 64 * kBiasBytes;
+static_assert(2 * sizeof(KTile) + 2 * sizeof(VTile) <= kPoolBytes, "FP32 tiles fit the pool");
+
+// v_mfma_f32_32x32x2_f32: A[row][k] in lane row + 32 k, B[k][col] in lane col + 32 k,
+// result in the 32x32 layout (common.hpp).
+__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
 
 // The rows of this lane's query in plain FP32, two passes over the keys: for
 // work-groups with a non-finite operand, and for bias rows so far apart that
@@ -111,11 +158,213 @@ __device__ __forceinline__ void attend_scalar(const AttnArgs& a, int b, int h, i
   for (int i = 0; i < 16; ++i) a.out[row * kHeadDim + 16 * half + i] = o[i] / l;
 }
 
+// The work-group's rows on the FP32 matrix cores, for operands whose range the
+// planes do not hold.  K and V^T tiles are staged in `pool` (double buffers, one
+// barrier per tile), each a tile ahead in registers; the bias is loaded a tile
+// ahead into the registers its logits take.  On gfx950 an FP32 MFMA and VALU
+// work never overlap, so each tile runs S^T, softmax and O^T += V^T P^T in
+// order.  Logits, reference and weights are those of the planes' path, with
+// the reference snapped to 0 while the row's largest logit lies within kSnap,
+// and moved when the running sum passes kSumLimit.
+__device__ __forceinline__ void attend_f32(const AttnArgs& a, int b, int h, int jq, int nkt,
+                                           uint8_t* pool) {
+  KTile* const Ks = reinterpret_cast<KTile*>(pool);
+  VTile* const Vs = reinterpret_cast<VTile*>(pool + 2 * sizeof(KTile));
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int half = lane >> 5;
+  const int l32 = lane & 31;
+  const int row8 = tid >> 3;         // key of the thread's K and V loads
+  const int col4 = (tid & 7) * 4;    // and their channels
+  const int last = nkt - 1;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  const int64_t head = ((int64_t)b * a.n * kHeads + h) * kHeadDim;
+
+  int found = a.mbias == nullptr;
+  if (!found) {
+    for (int k = tid; k < a.n; k += kThreads) found |= a.mbias[(int64_t)b * a.mb_stride + k] == 0.0f;
+  }
+  // the barrier also releases the pool
+  const bool has_unmasked = __syncthreads_or(found) != 0;
+
+  auto rows = [&](const float* base, int t) -> f32x4 {
+    const int key = t * kBk + row8;
+    return key < a.n ? *(const f32x4*)(base + head + (int64_t)key * kHidden + col4) : zero;
+  };
+  auto put = [&](int stage, f32x4 k, f32x4 v) {
+    *(f32x4*)&Ks[stage][row8][col4] = k;
+    Vs[stage][col4 + 0][row8] = v.x;
+    Vs[stage][col4 + 1][row8] = v.y;
+    Vs[stage][col4 + 2][row8] = v.z;
+    Vs[stage][col4 + 3][row8] = v.w;
+  };
+  const bool ok = jq < a.n;
+  const float* const brow = a.bias + ((int64_t)h * a.bias_rows + (ok ? jq : 0)) * a.bias_stride;
+  auto bias = [&](int t) -> f32x16 {
+    f32x4 x[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) {
+      const int key = t * kBk + 8 * rr + 4 * half;  // n % 4 == 0: all four in or out
+      x[rr] = ok && key < a.n ? *(const f32x4*)(brow + key) : zero;
+    }
+    return cat4(x[0], x[1], x[2], x[3]);
+  };
+
+  // Q, the B operand of S^T = K Q^T: lane holds Q[jq][16 half + s].
+  float qf[16];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 v =
+        ok ? *(const f32x4*)(a.q + head + (int64_t)jq * kHidden + 16 * half + 4 * i) : zero;
+    qf[4 * i + 0] = v.x;
+    qf[4 * i + 1] = v.y;
+    qf[4 * i + 2] = v.z;
+    qf[4 * i + 3] = v.w;
+  }
+
+  f32x16 o = {};
+  float l_run = 0.f;
+  auto run = [&](auto exact_tag) {
+    constexpr bool kExact = decltype(exact_tag)::value;
+    float m_ref = -INFINITY;  // largest tile max when the reference was last looked at
+    float c_ref = 0.f;        // the reference, in log2 units
+    bool has_ref = false;     // uniform per wave, as big
+    bool big = false;
+    // As in the planes' path, fast rows round logits past 2^22 (big) to log2
+    // units before the reference is taken off.
+    auto weights = [&](f32x16& x) {
+      if (big) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float y = x[r] * kLog2e;
+          x[r] = exp2_fast(y - c_ref);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref));
+      }
+    };
+    auto rescale = [&](float alpha) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] *= alpha;
+      l_run *= alpha;
+    };
+    // Logits x in natural units -> weights, in place.
+    auto softmax = [&](f32x16& x) {
+      if (kExact) {
+        const float mt = xor32_max(max16(x));
+        if (__any(mt > m_ref + kRescaleNat)) {
+          const float m_new = __builtin_elementwise_maximum(m_ref, mt);
+          const float c_new = m_new == -INFINITY ? 0.f : m_new * kLog2e;
+          rescale(m_ref == -INFINITY ? 0.f : exp2_fast(c_ref - c_new));
+          m_ref = m_new;
+          c_ref = c_new;
+        }
+        weights(x);
+        l_run += sum16(x);
+        return;
+      }
+      float ovf = 0.f;
+      if (has_ref) {
+        f32x16 p = x;
+        weights(p);
+        const float l_new = l_run + sum16(p);
+        const bool over = !(l_new <= kSumLimit);  // NaN or inf count as overflow
+        if (!__any(over)) {
+          l_run = l_new;
+          x = p;
+          return;
+        }
+        ovf = over ? 1.f : 0.f;
+      }
+      // Rare, taken by the whole wavefront.  A lane moves its reference only
+      // when it has none yet, when its own running sum overflowed, or when
+      // this tile's max lies more than kSnap above the reference; the decision
+      // is shared by the lane pair (l, l ^ 32) that holds the query.  After a
+      // sum overflow the true row max is at least c_ref + 52, so the reference
+      // moves up by at least kLift and the weights stay below 2^24.
+      const float mt = xor32_max(max16(x)) * kLog2e;
+      const bool fresh = m_ref == -INFINITY;
+      const bool need = fresh || xor32_max(ovf) > 0.f || mt > c_ref + kSnap;
+      m_ref = __builtin_elementwise_maximum(m_ref, mt);
+      const float snapped =
+          (m_ref == -INFINITY || (m_ref >= -kSnap && m_ref <= kSnap)) ? 0.f : m_ref;
+      const float c_new = fresh ? snapped
+                          : need ? __builtin_elementwise_maximum(snapped, c_ref + kLift)
+                                 : c_ref;
+      rescale(fresh ? 0.f : exp2_fast(c_ref - c_new));  // 1 when unchanged
+      c_ref = c_new;
+      has_ref = __all(m_ref != -INFINITY);
+      big = __any(!(__builtin_fabsf(c_ref) < kBigLogit));
+      weights(x);
+      l_run += sum16(x);
+    };
+
+    f32x16 x = bias(0);
+    put(0, rows(a.k, 0), rows(a.v, 0));
+    f32x4 kx = rows(a.k, min(1, last)), vx = rows(a.v, min(1, last));
+    __syncthreads();
+    for (int t = 0; t <= last; ++t) {
+      const int par = t & 1;
+      f32x16 s = {};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x4 kv = *(const f32x4*)&Ks[par][l32][16 * half + 4 * i];
+        s = mfma_f32(kv.x, qf[4 * i + 0], s);
+        s = mfma_f32(kv.y, qf[4 * i + 1], s);
+        s = mfma_f32(kv.z, qf[4 * i + 2], s);
+        s = mfma_f32(kv.w, qf[4 * i + 3], s);
+      }
+      if (a.mbias != nullptr || (t + 1) * kBk > a.n) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = t * kBk + mfma_row(r, half);
+          const float m =
+              key < a.n ? (a.mbias ? a.mbias[(int64_t)b * a.mb_stride + key] : 0.f) : -INFINITY;
+          s[r] = (s[r] + m) + x[r];  // the native order
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] += x[r];
+      }
+      x = bias(min(t + 1, last));
+      softmax(s);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const f32x4 vv = *(const f32x4*)&Vs[par][l32][8 * rr + 4 * half];
+        o = mfma_f32(vv.x, s[4 * rr + 0], o);
+        o = mfma_f32(vv.y, s[4 * rr + 1], o);
+        o = mfma_f32(vv.z, s[4 * rr + 2], o);
+        o = mfma_f32(vv.w, s[4 * rr + 3], o);
+      }
+      put(par ^ 1, kx, vx);  // the stage every wave left behind at the last barrier
+      kx = rows(a.k, min(t + 2, last));
+      vx = rows(a.v, min(t + 2, last));
+      __syncthreads();
+    }
+  };
+  if (has_unmasked)
+    run(std::false_type{});
+  else
+    run(std::true_type{});
+
+  const float l_tot = xor32_sum(l_run);
+  if (!ok) return;
+#pragma unroll
+  for (int rr = 0; rr < 4; ++rr)
+    *(f32x4*)(a.out + head + (int64_t)jq * kHidden + 8 * rr + 4 * half) =
+        f32x4{o[4 * rr + 0] / l_tot, o[4 * rr + 1] / l_tot, o[4 * rr + 2] / l_tot,
+              o[4 * rr + 3] / l_tot};
+}
+
 __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int nqt, int nkt,
                                                                 uint32_t total, int ppg) {
-  __shared__ __attribute__((aligned(16))) uint8_t kv[2][kTileBytes];
-  __shared__ __attribute__((aligned(16))) uint8_t bias_lds[kThreads / 64][kBiasBytes];
-  // each wave's largest |K| and |V| of tile t at [t & 1]; [2]: its largest |q|
+  __shared__ __attribute__((aligned(16))) uint8_t pool[kPoolBytes];
+  uint8_t (*const kv)[kTileBytes] = reinterpret_cast<uint8_t (*)[kTileBytes]>(pool);
+  uint8_t (*const bias_lds)[kBiasBytes] =
+      reinterpret_cast<uint8_t (*)[kBiasBytes]>(pool + 2 * kTileBytes);
+  // each wave's largest |K| and |V| of tile t at [t & 1]; [2]: its largest |q|, and look's answer
   __shared__ float red[3][kThreads / 64][2];
 
   int b, h, qt;
@@ -130,9 +379,10 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
   const int jq = j0 + l32;
   const int last = nkt - 1;
 
-  // The planes path; false (uniform) when the rows need attend_scalar.
-  auto attend = [&]() -> bool {
-    if (a.bias_stride > kMaxBiasStride) return false;
+  // The planes path; else (uniform) the path that serves the rows.
+  enum { kDone, kF32, kScalar };
+  auto attend = [&]() -> int {
+    if (a.bias_stride > kMaxBiasStride) return kScalar;
 
     // Row classification.  masked(t): some key of tile t has a nonzero mask
     // bias.  has_unmasked: some key k < n of the row has a zero mask bias.
@@ -187,8 +437,12 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
           __builtin_elementwise_maximum(__builtin_fabsf(x.x), __builtin_fabsf(x.y)),
           __builtin_elementwise_maximum(__builtin_fabsf(x.z), __builtin_fabsf(x.w)));
     };
+    float q_max;        // the work-group's largest |q|
+    float c_max = 0.f;  // this thread's largest |V|, all of channel vc
     auto note_max = [&](const f32x4& kx, const f32x4& vx, int slot) {
-      const float mk = wave_max(max4(kx)), mv = wave_max(max4(vx));
+      const float v4 = max4(vx);
+      c_max = __builtin_elementwise_maximum(c_max, v4);
+      const float mk = wave_max(max4(kx)), mv = wave_max(v4);
       if (lane == 0) {
         red[slot][w][0] = mk;
         red[slot][w][1] = mv;
@@ -202,6 +456,68 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         mk = __builtin_elementwise_maximum(mk, red[slot][i][0]);
         mv = __builtin_elementwise_maximum(mv, red[slot][i][1]);
       }
+    };
+    // Q planes (B operand of S^T = K Q^T): lane holds Q[jq][16 m + 8 half + e].
+    bf16x8 qh[2], ql[2];
+    int eq, ek, ev;  // plane exponents of the wave's q, of the tile's K, and E
+    // Whether no row or channel of the wave's q (its hi plane) lies below
+    // kEvenShare of its largest value, and no nonzero row or channel of K, over
+    // the eight keys of the tile (kx, largest |K| mk) that the wave holds.
+    auto q_even = [&]() -> bool {
+      f16x8 x[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        f32x4 bits = __builtin_bit_cast(f32x4, qh[m]);
+        asm volatile("" : "+v"(bits));  // formed here, not ahead of the loop in registers it needs
+        x[m] = __builtin_bit_cast(f16x8, bits);
+      }
+      auto at = [&](int i) { return __builtin_fabsf((float)x[i >> 3][i & 7]); };
+      float row = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) row = __builtin_elementwise_maximum(row, at(i));
+      row = xor32_max(row);
+      const float least = kEvenShare * wave_max(row);
+      bool bad = row < least;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) bad |= half_max(at(i)) < least;
+      return !__any(bad);
+    };
+    auto k_even = [&](const f32x4& kx, float mk) -> bool {
+      const float least = kEvenShare * mk;
+      float row = max4(kx);
+      row = __builtin_elementwise_maximum(row, dpp<0xB1>(row));
+      row = __builtin_elementwise_maximum(row, dpp<0x4E>(row));
+      row = __builtin_elementwise_maximum(row, dpp<0x141>(row));
+      bool bad = row != 0.f && row < least;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // lanes of equal lane % 8: row_ror:8, row and half swaps
+        float c = __builtin_fabsf(kx[e]);
+        c = __builtin_elementwise_maximum(c, dpp<0x128>(c));
+        const auto r = __builtin_amdgcn_permlane16_swap(
+            __builtin_bit_cast(unsigned, c), __builtin_bit_cast(unsigned, c), false, false);
+        c = xor32_max(__builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)r[0]),
+                                                    __builtin_bit_cast(float, (unsigned)r[1])));
+        bad |= c != 0.f && c < least;
+      }
+      return !__any(bad);
+    };
+    // Whether a tile of these maxima needs no look at its values (false for NaN),
+    // and the path for one that does (apart: V's scale is kMaxSpread off the
+    // other tiles').  Uniform.
+    auto plain = [&](float mk, float mv) { return q_max * mk <= kMaxProduct && mv < INFINITY; };
+    int q_known = -1;  // q_even() once it was needed; uniform per wave
+    auto look = [&](const f32x4& kx, float mk, float mv, bool apart) -> int {
+      if (!(mk < INFINITY && mv < INFINITY && q_max < INFINITY)) return kScalar;
+      if (apart || !(q_max * mk <= 0x1p96f)) return kF32;
+      if (q_known < 0) q_known = __builtin_amdgcn_readfirstlane(q_even());
+      const bool even = k_even(kx, mk) && q_known != 0;
+      // every wave's answer; a barrier ends the iteration before the next look
+      if (lane == 0) red[2][w][1] = even ? 0.f : 1.f;
+      __syncthreads();
+      float bad = 0.f;
+#pragma unroll
+      for (int i = 0; i < kThreads / 64; ++i) bad += red[2][i][1];
+      return bad != 0.f ? kF32 : kDone;
     };
     // A staged tile into planes: 16-byte chunk c of a plane's row r sits at
     // chunk c ^ swz(r).  V^T keys lie in the order of the S^T accumulator
@@ -221,7 +537,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
     };
     // plane_exp of a zero tile must not lower the smallest exponent
     auto value_exp = [](float m) -> int {
-      return __builtin_amdgcn_readfirstlane(m == 0.f ? 141 : plane_exp(m));
+      return __builtin_amdgcn_readfirstlane(m == 0.f ? kNoExp : plane_exp(m));
     };
     auto plane_rd = [&](int stage, int plane, int m) -> bf16x8 {
       return *(const bf16x8*)(kv[stage] + plane * kPlaneBytes + l32 * 64 +
@@ -260,9 +576,6 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       return cat4(x[0], x[1], x[2], x[3]);
     };
 
-    // Q planes (B operand of S^T = K Q^T): lane holds Q[jq][16 m + 8 half + e].
-    bf16x8 qh[2], ql[2];
-    int eq, ek, ev;  // plane exponents of the wave's q, of the tile's K, and E
     f32x4 ka, va;
     {
       const float* src = a.q + (((int64_t)b * a.n + min(jq, a.n - 1)) * kHeads + h) * kHeadDim + 8 * half;
@@ -290,14 +603,22 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       clip_kv(last < 1 ? last : 1, ka, va);
       note_max(k0, v0, 0);
       note_max(ka, va, 1);
-      if (lane == 0) red[2][w][0] = red[2][w][1] = mq;
+      if (lane == 0) red[2][w][0] = mq;
       __syncthreads();
-      float mk, mv, q0, q1;
+      float mk, mv;
       read_max(0, mk, mv);
-      read_max(2, q0, q1);
-      if (!(mk < INFINITY && mv < INFINITY && q0 < INFINITY)) {  // uniform; NaN too
-        wait_vmcnt<0>();  // no copy in flight when the LDS is released
-        return false;
+      q_max = red[2][0][0];
+#pragma unroll
+      for (int i = 1; i < kThreads / 64; ++i)
+        q_max = __builtin_elementwise_maximum(q_max, red[2][i][0]);
+      q_max = __builtin_bit_cast(
+          float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, q_max)));
+      if (!plain(mk, mv)) {
+        const int way = look(k0, mk, mv, false);
+        if (way != kDone) {
+          wait_vmcnt<0>();  // no copy in flight when the LDS is released
+          return way;
+        }
       }
       ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
       ev = value_exp(mv);
@@ -307,7 +628,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
 
     f32x16 o = {};
     float l_run = 0.f;
-    bool bad = false;  // a non-finite tile; uniform
+    int way = kDone;  // uniform
     auto run = [&](auto exact_tag) {
       constexpr bool kExact = decltype(exact_tag)::value;
       const f32x16 zero16 = {};
@@ -400,12 +721,15 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         if (t < last) {
           float mk, mv;
           read_max(par ^ 1, mk, mv);
-          if (!(mk < INFINITY && mv < INFINITY)) {  // uniform; NaN too
-            bad = true;
-            break;
+          const int et = value_exp(mv);
+          const bool apart =
+              et != kNoExp && ev != kNoExp && (et - ev > kMaxSpread || ev - et > kMaxSpread);
+          if (__builtin_expect(apart || !plain(mk, mv), 0)) {
+            way = look(ka, mk, mv, apart);
+            if (way != kDone) break;
           }
           ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
-          e_new = min(ev, value_exp(mv));
+          e_new = min(ev, et);
           put(par ^ 1, ka, va, ek, e_new);
         }
         load_kv(t + 2 <= last ? t + 2 : last, ka, va);
@@ -468,9 +792,33 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       run(std::true_type{});
     }
     wait_vmcnt<0>();  // no copy in flight when the LDS is released
-    if (bad) return false;
+    if (way != kDone) return way;
 
     const float l_tot = xor32_sum(l_run);
+    if (ev != kNoExp) {  // uniform: V is not all zero
+      // The shares of the file comment, decided alike by every wave.  The
+      // wave's bias fragment is free.
+      float top = 0.f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(o[r]));
+      top = xor32_max(top);
+      const float share =
+          __builtin_fmaf(kRowShare, l_tot, kWeightShare * __builtin_sqrtf((float)a.n));
+      // a NaN top or l_tot stays; l_tot is 0 where every logit is -inf
+      const bool low = __any(jq < a.n && l_tot != 0.f && top < share);
+      const float mine = xor32_max(c_max);  // both halves the same value
+      reinterpret_cast<f32x2*>(bias_lds[w])[l32] = f32x2{mine, low ? 1.f : 0.f};
+      __syncthreads();
+      f32x2 c = {};
+#pragma unroll
+      for (int i = 0; i < kThreads / 64; ++i) {
+        const f32x2 u = reinterpret_cast<const f32x2*>(bias_lds[i])[l32];
+        c.x = __builtin_elementwise_maximum(c.x, u.x);
+        c.y += u.y;
+      }
+      const float scaled = __builtin_ldexpf(c.x, ev);
+      if (__any(c.y != 0.f || (c.x != 0.f && scaled < 1.0f))) return kF32;
+    }
     if (jq < a.n) {
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
@@ -482,9 +830,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         *(f32x4*)(a.out + (((int64_t)b * a.n + jq) * kHeads + h) * kHeadDim + c) = ov;
       }
     }
-    return true;
+    return kDone;
   };
-  if (!attend()) attend_scalar(a, b, h, jq, half);
+  const int way = attend();
+  if (way == kScalar) attend_scalar(a, b, h, jq, half);
+  if (way == kF32) attend_f32(a, b, h, jq, nkt, pool);
 }
 
 }  // namespace

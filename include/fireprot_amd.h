@@ -173,7 +173,8 @@ int fpx_attn_core(float* q, float* k, float* v, float* bias, float* out, int bat
  * reference's vector_bias1000 entry does (fireprot_ck_attention.cpp:106-107);
  * the computation is FP32-accurate on the 16-bit matrix cores (operands split
  * into power-of-two scaled fp16 planes in the kernel; plain FP32 where q, k or
- * v is not finite), asynchronous on the caller's stream, with no allocation. */
+ * v is not finite, or spans more binary orders than the planes hold),
+ * asynchronous on the caller's stream, with no allocation. */
 int ck_attention(float* q, float* k, float* v, float* bias, float* out, int batch, int n,
                  void* stream);
 int ck_attention_exact1536(float* q, float* k, float* v, float* bias, float* out, int batch,
