@@ -44,13 +44,12 @@
 //
 // A row whose logits are all -inf gives NaN, as torch.softmax does.  fp16
 // planes cannot carry an infinity beside finite values (its residual is NaN),
-// so a work-group that meets a non-finite q, k or v computes its rows in plain
-// FP32 (attend_scalar) with the native propagation.
+// so a work-group that meets a non-finite q, k or v computes its rows on the
+// FP32 matrix cores (attend_f32) with the native propagation.
 //
 // Range.  A plane pair resolves 2^-25 in scaled units, 2^-39 of the largest
 // value it is scaled with, whereas FP32 keeps 24 bits of every value.  A
-// work-group whose operands need more runs on the FP32 matrix cores
-// (attend_f32):
+// work-group whose operands need more runs on attend_f32 as well:
 //   - logits: what the planes drop of one logit is at most 32 products of one
 //     operand's largest value and the other's resolution, for both operands:
 //     64 2^-39 max|q| max|K| = 2^-33 max|q| max|K|.  Up to max|q| max|K| =
@@ -72,7 +71,9 @@
 // are the usual cause) go to FP32 as they are met.  So the planes' error is
 // relative to the largest output of the row and to the largest V of the
 // channel.  The looks cost 1.3% at N = 1536 (3118 to 3160 us) and at most
-// 0.6 us of 13 at N = 128.
+// 0.7 us of 13 at N = 128.  attend_f32 runs at the rate of a kernel of its own
+// (B = 64, N = 1536: 786 us for a NaN in the first tile, 406 on the planes); a
+// value or range that only the last tiles or the sums show costs both, 1.2 ms.
 //
 // Bound: VALU issue beside the matrix cores (about 170 VALU instructions and
 // 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.23 ms; on the FP32
@@ -118,48 +119,9 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
-// The rows of this lane's query in plain FP32, two passes over the keys: for
-// work-groups with a non-finite operand, and for bias rows so far apart that
-// a wave's 32 span more than 4 GB.  Lane half `half` holds channels
-// 16 half .. + 15 of the query and of the output.
-__device__ __forceinline__ void attend_scalar(const AttnArgs& a, int b, int h, int jq, int half) {
-  const bool ok = jq < a.n;
-  const int64_t row = ((int64_t)b * a.n + (ok ? jq : 0)) * kHeads + h;
-  float q[16], o[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    q[i] = a.q[row * kHeadDim + 16 * half + i];
-    o[i] = 0.f;
-  }
-  const float* bias = a.bias + ((int64_t)h * a.bias_rows + (ok ? jq : 0)) * a.bias_stride;
-  auto logit = [&](int key) -> float {
-    const float* k = a.k + (((int64_t)b * a.n + key) * kHeads + h) * kHeadDim + 16 * half;
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s = __builtin_fmaf(q[i], k[i], s);
-    s = xor32_sum(s);
-    const float m = a.mbias ? a.mbias[(int64_t)b * a.mb_stride + key] : 0.f;
-    return (s + m) + bias[key];
-  };
-  float m = -INFINITY;
-#pragma unroll 1
-  for (int key = 0; key < a.n; ++key) m = __builtin_elementwise_maximum(m, logit(key));
-  float l = 0.f;
-#pragma unroll 1
-  for (int key = 0; key < a.n; ++key) {
-    const float p = exp2_fast((logit(key) - m) * kLog2e);
-    l += p;
-    const float* v = a.v + (((int64_t)b * a.n + key) * kHeads + h) * kHeadDim + 16 * half;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[i] = __builtin_fmaf(p, v[i], o[i]);
-  }
-  if (!ok) return;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) a.out[row * kHeadDim + 16 * half + i] = o[i] / l;
-}
-
-// The work-group's rows on the FP32 matrix cores, for operands whose range the
-// planes do not hold.  K and V^T tiles are staged in `pool` (double buffers, one
+// The work-group's rows on the FP32 matrix cores, for operands that the planes
+// do not hold, and for bias rows so far apart that a wave's 32 span more than
+// 4 GB.  K and V^T tiles are staged in `pool` (double buffers, one
 // barrier per tile), each a tile ahead in registers; the bias is loaded a tile
 // ahead into the registers its logits take.  On gfx950 an FP32 MFMA and VALU
 // work never overlap, so each tile runs S^T, softmax and O^T += V^T P^T in
@@ -366,6 +328,10 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       reinterpret_cast<uint8_t (*)[kBiasBytes]>(pool + 2 * kTileBytes);
   // each wave's largest |K| and |V| of tile t at [t & 1]; [2]: its largest |q|, and look's answer
   __shared__ float red[3][kThreads / 64][2];
+  // largest |V| so far (float bits) of channel l32, a cell for each lane half at the
+  // plane reads' offsets, whose address register it shares
+  __shared__ __attribute__((aligned(16))) uint8_t channels[kPlaneBytes];
+  __shared__ uint32_t low_rows;  // some query's output is below its share
 
   int b, h, qt;
   attn_item(blockIdx.x, total, a.batch, nqt, ppg, b, h, qt);
@@ -379,10 +345,13 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
   const int jq = j0 + l32;
   const int last = nkt - 1;
 
-  // The planes path; else (uniform) the path that serves the rows.
-  enum { kDone, kF32, kScalar };
-  auto attend = [&]() -> int {
-    if (a.bias_stride > kMaxBiasStride) return kScalar;
+  // The planes' path; false (uniform) when the rows need attend_f32.
+  auto attend = [&]() -> bool {
+    if (a.bias_stride > kMaxBiasStride) return false;
+    const uint32_t rd0 = l32 * 64 + 16 * (half ^ swz(l32));
+    auto channel_max = [&]() { return reinterpret_cast<uint32_t*>(channels + rd0); };
+    if (w == 0) *channel_max() = 0u;
+    if (tid == 0) low_rows = 0u;
 
     // Row classification.  masked(t): some key of tile t has a nonzero mask
     // bias.  has_unmasked: some key k < n of the row has a zero mask bias.
@@ -437,11 +406,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
           __builtin_elementwise_maximum(__builtin_fabsf(x.x), __builtin_fabsf(x.y)),
           __builtin_elementwise_maximum(__builtin_fabsf(x.z), __builtin_fabsf(x.w)));
     };
-    float q_max;        // the work-group's largest |q|
-    float c_max = 0.f;  // this thread's largest |V|, all of channel vc
+    float q_max;  // the work-group's largest |q|
     auto note_max = [&](const f32x4& kx, const f32x4& vx, int slot) {
-      const float v4 = max4(vx);
-      c_max = __builtin_elementwise_maximum(c_max, v4);
+      const float v4 = max4(vx);  // four keys of channel vc
+      __hip_atomic_fetch_max(channel_max(), __builtin_bit_cast(uint32_t, v4), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
       const float mk = wave_max(max4(kx)), mv = wave_max(v4);
       if (lane == 0) {
         red[slot][w][0] = mk;
@@ -502,13 +471,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       return !__any(bad);
     };
     // Whether a tile of these maxima needs no look at its values (false for NaN),
-    // and the path for one that does (apart: V's scale is kMaxSpread off the
-    // other tiles').  Uniform.
+    // and whether one that does fits the planes.  Uniform.
     auto plain = [&](float mk, float mv) { return q_max * mk <= kMaxProduct && mv < INFINITY; };
     int q_known = -1;  // q_even() once it was needed; uniform per wave
-    auto look = [&](const f32x4& kx, float mk, float mv, bool apart) -> int {
-      if (!(mk < INFINITY && mv < INFINITY && q_max < INFINITY)) return kScalar;
-      if (apart || !(q_max * mk <= 0x1p96f)) return kF32;
+    auto look = [&](const f32x4& kx, float mk, float mv) -> bool {
+      if (!(mk < INFINITY && mv < INFINITY && q_max * mk <= 0x1p96f)) return false;
       if (q_known < 0) q_known = __builtin_amdgcn_readfirstlane(q_even());
       const bool even = k_even(kx, mk) && q_known != 0;
       // every wave's answer; a barrier ends the iteration before the next look
@@ -517,21 +484,25 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       float bad = 0.f;
 #pragma unroll
       for (int i = 0; i < kThreads / 64; ++i) bad += red[2][i][1];
-      return bad != 0.f ? kF32 : kDone;
+      return bad == 0.f;
     };
     // A staged tile into planes: 16-byte chunk c of a plane's row r sits at
     // chunk c ^ swz(r).  V^T keys lie in the order of the S^T accumulator
     // registers: key group g of four at position 16 (g / 4) + 4 (0, 2, 1,
     // 3)[g % 4].
     const uint32_t kput = kkey * 64 + 16 * ((kc4 >> 3) ^ swz(kkey)) + (kc4 & 4) * 2;
-    const int vpos = (vg >> 2) * 16 + ((vg & 1) * 2 + ((vg >> 1) & 1)) * 4;
-    const uint32_t vput = vc * 64 + 16 * ((vpos >> 3) ^ swz(vc)) + (vpos & 7) * 2;
     auto put = [&](int stage, const f32x4& kx, const f32x4& vx, int ek, int ev) {
       bf16x4 hi, lo;
       split_f16(ldexp4(kx, ek), hi, lo);
       *(bf16x4*)(kv[stage] + kput) = hi;
       *(bf16x4*)(kv[stage] + kPlaneBytes + kput) = lo;
       split_f16(ldexp4(vx, ev), hi, lo);
+      // vg = 2 w + half: its four keys start at position 16 (w / 2) + 8 half +
+      // 4 (w % 2), half w % 2 of the chunk that plane_rd(.., m = w / 2) reads.
+      // Formed from that offset here: there is no register to hold it.
+      uint32_t flip = 32u * (w >> 1);
+      asm volatile("" : "+s"(flip));
+      const uint32_t vput = (rd0 ^ flip) + 8 * (w & 1);
       *(bf16x4*)(kv[stage] + 2 * kPlaneBytes + vput) = hi;
       *(bf16x4*)(kv[stage] + 3 * kPlaneBytes + vput) = lo;
     };
@@ -540,8 +511,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       return __builtin_amdgcn_readfirstlane(m == 0.f ? kNoExp : plane_exp(m));
     };
     auto plane_rd = [&](int stage, int plane, int m) -> bf16x8 {
-      return *(const bf16x8*)(kv[stage] + plane * kPlaneBytes + l32 * 64 +
-                              16 * ((2 * m + half) ^ swz(l32)));
+      return *(const bf16x8*)(kv[stage] + plane * kPlaneBytes + (rd0 ^ (32 * m)));
     };
 
     // Bias fragment of tile t: instruction i copies rows 8 i + lane / 8 of the
@@ -613,12 +583,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         q_max = __builtin_elementwise_maximum(q_max, red[2][i][0]);
       q_max = __builtin_bit_cast(
           float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, q_max)));
-      if (!plain(mk, mv)) {
-        const int way = look(k0, mk, mv, false);
-        if (way != kDone) {
-          wait_vmcnt<0>();  // no copy in flight when the LDS is released
-          return way;
-        }
+      q_max = __builtin_bit_cast(
+          float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, q_max)));
+      if (!plain(mk, mv) && !look(k0, mk, mv)) {
+        wait_vmcnt<0>();  // no copy in flight when the LDS is released
+        return false;
       }
       ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
       ev = value_exp(mv);
@@ -628,7 +597,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
 
     f32x16 o = {};
     float l_run = 0.f;
-    int way = kDone;  // uniform
+    bool fits = true;  // uniform
     auto run = [&](auto exact_tag) {
       constexpr bool kExact = decltype(exact_tag)::value;
       const f32x16 zero16 = {};
@@ -725,8 +694,8 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
           const bool apart =
               et != kNoExp && ev != kNoExp && (et - ev > kMaxSpread || ev - et > kMaxSpread);
           if (__builtin_expect(apart || !plain(mk, mv), 0)) {
-            way = look(ka, mk, mv, apart);
-            if (way != kDone) break;
+            fits = !apart && look(ka, mk, mv);
+            if (!fits) break;
           }
           ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
           e_new = min(ev, et);
@@ -792,12 +761,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       run(std::true_type{});
     }
     wait_vmcnt<0>();  // no copy in flight when the LDS is released
-    if (way != kDone) return way;
+    if (!fits) return false;
 
     const float l_tot = xor32_sum(l_run);
     if (ev != kNoExp) {  // uniform: V is not all zero
-      // The shares of the file comment, decided alike by every wave.  The
-      // wave's bias fragment is free.
+      // The shares of the file comment, decided alike by every wave.
       float top = 0.f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) top = __builtin_elementwise_maximum(top, __builtin_fabsf(o[r]));
@@ -805,19 +773,10 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       const float share =
           __builtin_fmaf(kRowShare, l_tot, kWeightShare * __builtin_sqrtf((float)a.n));
       // a NaN top or l_tot stays; l_tot is 0 where every logit is -inf
-      const bool low = __any(jq < a.n && l_tot != 0.f && top < share);
-      const float mine = xor32_max(c_max);  // both halves the same value
-      reinterpret_cast<f32x2*>(bias_lds[w])[l32] = f32x2{mine, low ? 1.f : 0.f};
+      if (jq < a.n && l_tot != 0.f && top < share) low_rows = 1u;
       __syncthreads();
-      f32x2 c = {};
-#pragma unroll
-      for (int i = 0; i < kThreads / 64; ++i) {
-        const f32x2 u = reinterpret_cast<const f32x2*>(bias_lds[i])[l32];
-        c.x = __builtin_elementwise_maximum(c.x, u.x);
-        c.y += u.y;
-      }
-      const float scaled = __builtin_ldexpf(c.x, ev);
-      if (__any(c.y != 0.f || (c.x != 0.f && scaled < 1.0f))) return kF32;
+      const float c = xor32_max(__builtin_bit_cast(float, *channel_max()));
+      if (low_rows != 0u || __any(c != 0.f && __builtin_ldexpf(c, ev) < 1.0f)) return false;
     }
     if (jq < a.n) {
 #pragma unroll
@@ -830,11 +789,9 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         *(f32x4*)(a.out + (((int64_t)b * a.n + jq) * kHeads + h) * kHeadDim + c) = ov;
       }
     }
-    return kDone;
+    return true;
   };
-  const int way = attend();
-  if (way == kScalar) attend_scalar(a, b, h, jq, half);
-  if (way == kF32) attend_f32(a, b, h, jq, nkt, pool);
+  if (!attend()) attend_f32(a, b, h, jq, nkt, pool);
 }
 
 }  // namespace

@@ -102,3 +102,29 @@ def test_bias_rows_beyond_32_bit_offsets():
     rows[:, :n] = bias.view(4 * n, n)
     out = _run(q, k, v, rows, row=row)
     torch.testing.assert_close(out, _torch(q, k, v, bias, None, torch.float32), atol=2e-6, rtol=0)
+
+
+def test_non_finite_inputs_cost_no_more_than_fp32_products():
+    """A batch whose every row holds a NaN runs on the FP32 matrix cores (1.8
+    times the planes' time at N = 1536), not key by key (over 20 times).  Three
+    times the finite time leaves room for noise."""
+    q, k, v, bias = _inputs(64, 512, 17)
+
+    def seconds():
+        for _ in range(2):
+            _run(q, k, v, bias)
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(10):
+            _run(q, k, v, bias)
+        end.record()
+        torch.cuda.synchronize()
+        return start.elapsed_time(end)
+
+    finite = min(seconds() for _ in range(3))
+    k[:, 300, 1, 5] = float("nan")
+    k[:, 300, 2, 5] = float("inf")
+    v[:, 300, 0::3, 5] = float("nan")
+    broken = min(seconds() for _ in range(3))
+    print(f"finite {finite:.3f} ms, non-finite {broken:.3f} ms", flush=True)
+    assert broken <= 3.0 * finite, (broken, finite)
