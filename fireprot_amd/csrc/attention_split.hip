@@ -36,7 +36,7 @@
 //     would pass 2^15;
 //     P' = exp2(x - (c + g_t)) with the tile's exponent shift g_t folded into
 //     the exact integer c + g_t.  The block's bias copy is stored relative
-//     to each query's reference (bias_reference_kernel): the reference then
+//     to each query's reference (pair_bias_kernel): the reference then
 //     starts at 0, and while it and g_t stay 0 the weights are exp2(x);
 //   exact (fully masked rows, and rows whose logits are not bounded):
 //     fl(fl(s + mask) + bias) in natural units, as the native path rounds
@@ -1174,7 +1174,7 @@ void attention_const_kernel(AttnArgs a, int nqt, int nkt, int nchunks, uint32_t 
   const int hq0 = xcd * nhq / kXcds;
   const int nh = (xcd + 1) * nhq / kXcds - hq0;
   if (nh == 0) return;
-  if (LAYOUT == kAttnBlock && a.const_m != nullptr) {
+  if constexpr (LAYOUT == kAttnBlock) {
     // The block's chunk list (pair_bias_kernel): a persistent grid, a
     // multiple of kXcds work-groups, walks it.
     const int count = (int)__builtin_amdgcn_readfirstlane(a.const_m[2]);
@@ -1185,15 +1185,15 @@ void attention_const_kernel(AttnArgs a, int nqt, int nkt, int nchunks, uint32_t 
       const_item<LAYOUT>(a, nqt, nkt, chunk, hq0 + slot % nh, ring, Sv);
       __syncthreads();
     }
-    return;
-  }
-  // Every (chunk, pair) item, one work-group each (the items without
-  // constant-mask rows leave at once).
-  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
-    const int slot = (int)(item / kXcds);
-    if (slot < nh * nchunks) {
-      const_item<LAYOUT>(a, nqt, nkt, slot / nh, hq0 + slot % nh, ring, Sv);
-      __syncthreads();
+  } else {
+    // Every (chunk, pair) item, one work-group each (the items without
+    // constant-mask rows leave at once).
+    for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+      const int slot = (int)(item / kXcds);
+      if (slot < nh * nchunks) {
+        const_item<LAYOUT>(a, nqt, nkt, slot / nh, hq0 + slot % nh, ring, Sv);
+        __syncthreads();
+      }
     }
   }
 }
@@ -1267,8 +1267,9 @@ __device__ __forceinline__ void row_norms(const AttnArgs& a, uint32_t* tile_flag
 // (equal quantised logits get equal weights), their sum l_q, and P 2^kVShift
 // split into fp16 planes in the P.V operand order, stored as the four
 // 16-byte parts of a bias fragment.  With no constant-mask row, const_m[0]
-// becomes a NaN (no row's m matches it).  Work-group 0 also counts the
-// chunks whose rows have that m (const_m[1]) and lists the others.
+// becomes a NaN (no row's m matches it).  Work-group 0 also lists the chunks of
+// another m, and counts both kinds (const_m[1], a record of how many chunks the
+// shared weights serve, is read by no kernel).
 constexpr int kBiasWaves = 8;
 template <bool kWeights>
 __global__ __launch_bounds__(kBiasWaves * 64) void pair_bias_kernel(AttnArgs a, float* bias_l2,
@@ -1453,7 +1454,9 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
   if (total == 0) return hipSuccess;
   if (total > 0x7fffffffull) return hipErrorInvalidValue;
   if (a.tile_flags == nullptr || a.bias_l2 == nullptr || a.scales == nullptr ||
-      nkt > kTileFlagWords * 32)
+      nkt > kTileFlagWords * 32 ||
+      (layout == kAttnBlock &&
+       (a.const_m == nullptr || a.const_l == nullptr || a.const_p == nullptr)))
     return hipErrorInvalidValue;
   const size_t mask_row_bytes = (size_t)nkt * kBk * sizeof(float);
   const int ppg = pair_group_size(nqt, (uint64_t)kBq * (uint64_t)a.np * sizeof(float));
@@ -1481,10 +1484,8 @@ hipError_t launch_attention_split(int layout, const AttnArgs& a, hipStream_t str
     // work-groups per CU) over their chunk list
     int cap = device_cu_count() * 2;
     cap -= cap % kXcds;
-    const uint32_t grid =
-        a.const_m != nullptr ? (uint32_t)std::max(cap, kXcds) : (uint32_t)const_items;
-    hipLaunchKernelGGL((attention_const_kernel<kAttnBlock>), dim3(grid), dim3(kThreads), 0, stream,
-                       a, nqt, nkt, nchunks, (uint32_t)const_items);
+    hipLaunchKernelGGL((attention_const_kernel<kAttnBlock>), dim3((uint32_t)std::max(cap, kXcds)),
+                       dim3(kThreads), 0, stream, a, nqt, nkt, nchunks, (uint32_t)const_items);
   } else if (layout == kAttnStaged) {
     hipLaunchKernelGGL((attention_split_kernel<kAttnStaged, false>), dim3((uint32_t)total),
                        dim3(kThreads), mask_row_bytes, stream, a, nqt, nkt, (uint32_t)total, ppg);

@@ -38,8 +38,8 @@ size_t elem_bytes(int dtype) { return dtype == FPX_BF16 ? 2 : 4; }
 //   kMagnitudeWords words of the magnitude record; scales [3][n][4][np / 32]
 //   float (the plane layout's per-tile inverse scales of q, k and v^T); FP32
 //   only: the constant-mask rows' weights and chunk list (AttnArgs::const_m,
-//   const_l, const_p: kConstListWord words and room for two lists of
-//   ceil(n / kConstRows) chunk indices, l [4][np] float, the planes
+//   const_l, const_p: kConstListWord words, the list in room for twice the
+//   ceil(n / kConstRows) chunk indices it may hold, l [4][np] float, the planes
 //   [4][np / 32][ceil(n / 32)] x 4 KB).
 // FP32 blocks hold q, k and v^T in the fp16 plane layout (ProjArgs), in the
 // same bytes as FP32 values.

@@ -110,14 +110,13 @@ struct AttnArgs {
   const uint32_t* tile_flags;
   const uint32_t* magnitudes;  // kAttnBlock: nullable; enables the trailing-tile skip
   const float* scales;  // kAttnBlock, kAttnStaged: the planes' inverse scales
-  // kAttnBlock, nullable: the constant-mask rows' shared weights and work
-  // list, written by launch_pair_bias: const_m[0] the mask bias m the weights
-  // serve (float bits; a NaN when no row has a constant mask), const_m[1] and
-  // const_m[2] the numbers of kConstRows-row chunks with constant-mask rows
-  // of that m and of another m, the latter's chunk indices from word
-  // kConstListWord; const_l[4][np] each query's weight sum, const_p the
-  // weights' fp16 planes, 4 KB per (head, 32-query tile, key tile).  Each may
-  // be null only with all.
+  // kAttnBlock (null in the other layouts): the constant-mask rows' shared
+  // weights and work list, written by launch_pair_bias: const_m[0] the mask
+  // bias m the weights serve (float bits; a NaN when no row has a constant
+  // mask), const_m[1] and const_m[2] the numbers of kConstRows-row chunks with
+  // constant-mask rows of that m (a record no kernel reads) and of another m,
+  // the latter's chunk indices from word kConstListWord; const_l[4][np] each query's weight sum, const_p the
+  // weights' fp16 planes, 4 KB per (head, 32-query tile, key tile).
   uint32_t* const_m;
   float* const_l;
   uint8_t* const_p;
@@ -365,7 +364,7 @@ struct TransitionArgs {
   const float* w_b;   // [512][128]
   const float* w_o;   // [128][512]
   // the 16 chunks' weight planes (fp16 bits, 768 KB), the folded biases
-  // [2][512] and the plane exponents (1156 ints, see transition.hip)
+  // [2][512] and the plane exponents (1188 ints, see transition.hip)
   __bf16* planes;
   float* fbias;
   int* exps;
