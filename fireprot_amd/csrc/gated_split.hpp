@@ -373,7 +373,7 @@ static __global__ __launch_bounds__(256) void row_max_zero_kernel(uint32_t* rowm
 // 128 rows 2 instead of 4 (55 against 58).  Past that its tiles, each of
 // another row, are slower to read and write than a row's run: N = 384 248 us
 // against 241, N = 777 1240 against 1210.
-constexpr int64_t kSpreadPairs = 1 << 17;  // N = 362
+constexpr int64_t kSpreadPairs = 1 << 17;  // rows x span: up to N = 352 (11 key runs)
 inline hipError_t launch_gated_split(const GatedArgs& a, hipStream_t stream) {
   const int tiles_k = a.span_k / kGatedRows;
   const int64_t ntiles = (int64_t)a.rows_r * tiles_k;

@@ -115,8 +115,9 @@ struct AttnArgs {
   // bias m the weights serve (float bits; a NaN when no row has a constant
   // mask), const_m[1] and const_m[2] the numbers of kConstRows-row chunks with
   // constant-mask rows of that m (a record no kernel reads) and of another m,
-  // the latter's chunk indices from word kConstListWord; const_l[4][np] each query's weight sum, const_p the
-  // weights' fp16 planes, 4 KB per (head, 32-query tile, key tile).
+  // the latter's chunk indices from word kConstListWord; const_l[4][np] each
+  // query's weight sum, const_p the weights' fp16 planes, 4 KB per (head,
+  // 32-query tile, key tile).
   uint32_t* const_m;
   float* const_l;
   uint8_t* const_p;

@@ -1,9 +1,9 @@
 """The triangle multiplication at the sizes where its projection's work split
 changes, and where the contraction's keys end inside a 128-key panel.
 
-On 256 CUs the projection deals whole rows (N = 96, 160, 256, 363), or tiles of
-all rows with atomic row maxima (N = 97, 128, 257, 300, 362); N = 33, 97, 129,
-257 and 363 end a key run of 32 after one key.  Sampled rows are held to
+On 256 CUs the projection deals whole rows (N = 33, 96, 160, 256, 353, 362, 363),
+or tiles of all rows with atomic row maxima (N = 97, 128, 129, 257, 300, 352, the
+largest); N = 33, 97, 129, 257 and 353 end a key run of 32 after one key.  Sampled rows are held to
 float64: the largest error within twice that of the same oracle in FP32 (or
 2e-6 of the largest value).  The workspace holds NaN, so a maximum or a tile
 left unwritten shows.
@@ -20,7 +20,7 @@ from oracle import triangle_multiplication as tm
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [33, 96, 97, 128, 129, 160, 256, 257, 300, 362, 363])
+@pytest.mark.parametrize("n", [33, 96, 97, 128, 129, 160, 256, 257, 300, 352, 353, 362, 363])
 @pytest.mark.parametrize("outgoing", [True, False])
 def test_work_split_edges(n, outgoing):
     print(f"case n={n} outgoing={outgoing}", flush=True)
