@@ -27,7 +27,7 @@
 // into accumulator order, each instruction touches 32 rows.
 //
 // Rows with at least one unmasked key (fast): logits fma(acc, 2^-(e_q+e_k),
-// bias) in natural units (plus the mask bias on masked tiles), weights
+// bias) in natural units (plus the mask bias where a mask is given), weights
 // P' = exp2(fma(x, log2(e), -c)) with one integer reference c per query, 7
 // below the ceiling of the largest logit when it was set: no max is formed
 // until a lane's 16 weights of a tile sum past 2^15 (or at the first tile).
@@ -70,15 +70,15 @@
 // Tiles of V further apart than 2^20 (kMaxSpread; padded keys holding anything
 // are the usual cause) go to FP32 as they are met.  So the planes' error is
 // relative to the largest output of the row and to the largest V of the
-// channel.  The looks cost 1.3% at N = 1536 (3118 to 3160 us) and at most
-// 0.7 us of 13 at N = 128.  attend_f32 runs at the rate of a kernel of its own
+// channel.  The looks cost 1.6% at N = 1536 (3080 to 3129 us) and at most
+// 0.6 us of 13 at N = 128.  attend_f32 runs at the rate of a kernel of its own
 // (B = 64, N = 1536: 786 us for a NaN in the first tile, 406 on the planes); a
 // value or range that only the last tiles or the sums show costs both, 1.2 ms.
 //
 // Bound: VALU issue beside the matrix cores (about 170 VALU instructions and
-// 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.23 ms; on the FP32
-// matrix cores, which never overlap with VALU work, 5.42 ms.  N = 384 175 us
-// against 287.
+// 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.13 ms; on the FP32
+// matrix cores, which never overlap with VALU work, 5.39 ms.  N = 384 176 us
+// against 304.
 #include "attn_common.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
@@ -353,8 +353,9 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
     if (w == 0) *channel_max() = 0u;
     if (tid == 0) low_rows = 0u;
 
-    // Row classification.  masked(t): some key of tile t has a nonzero mask
-    // bias.  has_unmasked: some key k < n of the row has a zero mask bias.
+    // Row classification.  masked(t): the mask bias is added to tile t's logits
+    // (every tile where a mask is given, zeros or not; the tile that ends past
+    // n).  has_unmasked: some key k < n of the row has a zero mask bias.
     int found = a.mbias == nullptr;
     if (!found) {
       for (int k = tid; k < a.n; k += kThreads) found |= a.mbias[(int64_t)b * a.mb_stride + k] == 0.0f;
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
     };
     // Whether a tile of these maxima needs no look at its values (false for NaN),
     // and whether one that does fits the planes.  Uniform.
-    auto plain = [&](float mk, float mv) { return q_max * mk <= kMaxProduct && mv < INFINITY; };
+    auto plain = [&](float mk, float mv) { return (q_max * mk <= kMaxProduct) & (mv < INFINITY); };
     int q_known = -1;  // q_even() once it was needed; uniform per wave
     auto look = [&](const f32x4& kx, float mk, float mv) -> bool {
       if (!(mk < INFINITY && mv < INFINITY && q_max * mk <= 0x1p96f)) return false;
@@ -506,9 +507,9 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       *(bf16x4*)(kv[stage] + 2 * kPlaneBytes + vput) = hi;
       *(bf16x4*)(kv[stage] + 3 * kPlaneBytes + vput) = lo;
     };
-    // plane_exp of a zero tile must not lower the smallest exponent
-    auto value_exp = [](float m) -> int {
-      return __builtin_amdgcn_readfirstlane(m == 0.f ? kNoExp : plane_exp(m));
+    // V's exponent of a tile; a zero tile keeps the one so far
+    auto value_exp = [](float m, int so_far) -> int {
+      return __builtin_amdgcn_readfirstlane(m == 0.f ? so_far : plane_exp(m));
     };
     auto plane_rd = [&](int stage, int plane, int m) -> bf16x8 {
       return *(const bf16x8*)(kv[stage] + plane * kPlaneBytes + (rd0 ^ (32 * m)));
@@ -590,7 +591,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         return false;
       }
       ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));
-      ev = value_exp(mv);
+      ev = value_exp(mv, kNoExp);
       put(0, k0, v0, ek, ev);
       __syncthreads();
     }
@@ -690,11 +691,10 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
         if (t < last) {
           float mk, mv;
           read_max(par ^ 1, mk, mv);
-          const int et = value_exp(mv);
-          const bool apart =
-              et != kNoExp && ev != kNoExp && (et - ev > kMaxSpread || ev - et > kMaxSpread);
-          if (__builtin_expect(apart || !plain(mk, mv), 0)) {
-            fits = !apart && look(ka, mk, mv);
+          const int et = value_exp(mv, ev);
+          const bool near = (unsigned)(et - ev + kMaxSpread) <= 2u * kMaxSpread;
+          if (__builtin_expect(!(near & plain(mk, mv)), 0)) {
+            fits = (near || ev == kNoExp) && (plain(mk, mv) || look(ka, mk, mv));
             if (!fits) break;
           }
           ek = __builtin_amdgcn_readfirstlane(plane_exp(mk));

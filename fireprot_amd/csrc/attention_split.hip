@@ -378,7 +378,7 @@ __device__ __forceinline__ void attend_item(const AttnArgs& a, int nqt, int nkt_
   const bool live = j0 + 32 * w < a.n;  // uniform per wave
 
   // Per-work-group buffer descriptors over the (b, h) slices and the wave's
-  // bias fragments (h, qt32, all key tiles), as in the FP32 kernel.
+  // bias fragments (h, qt32, all key tiles).
   const int64_t bh = (int64_t)b * kHeads + h;
   const int64_t nt = a.np >> 5;
   const int64_t frag = ((int64_t)h * nt + qt32) * nt * 1024;

@@ -1,6 +1,6 @@
 // BF16-storage / FP32-accumulate variant of the triangle-attention block.
 //
-// Same dataflow as the FP32 block (projection.hip, attention.hip) with every
+// Same dataflow as the FP32 block (projection.hip, attention_split.hip) with every
 // stored tensor in bf16 -- z, weights, q, k, v^T, the sigmoid gate, the
 // triangle bias, the gated output and dz -- and all accumulation, LayerNorm
 // statistics and softmax arithmetic in FP32 on the gfx950 instruction
@@ -315,7 +315,7 @@ hipError_t launch_proj_mode(const Bf16ProjArgs& a, hipStream_t stream, int wgs_p
 //     the bytes per tile, and the kernel then waits on its loads).
 //   - q and the bias copy are stored scaled by log2(e), so the logits leave
 //     the matrix cores in log2 units.
-//   - Rows with an unmasked key: p = exp2(x - c) with the FP32 kernels'
+//   - Rows with an unmasked key: p = exp2(x - c) with a
 //     snapped reference c (0 while the row max lies within kSnap of it;
 //     rescaled only when a running sum passes kSumLimit), so a tile needs no
 //     max, no cross-lane exchange and no branch, and while every reference
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_bf16_kernel(Bf16AttnArg
       }
     };
 
-    // Reference state of this lane's query (log2 units; see attention.hip).
+    // Reference state of this lane's query (log2 units; see attend_f32).
     float m_ref = -INFINITY;
     float m_thr = -INFINITY;
     float c_ref = 0.f;
@@ -541,7 +541,7 @@ __global__ __launch_bounds__(kThreads, 3) void attention_bf16_kernel(Bf16AttnArg
         }
         ovf = over ? 1.f : 0.f;
       }
-      // Rare path, taken by the whole wavefront (attention.hip), in log2 units.
+      // Rare path, taken by the whole wavefront (as in attend_f32), in log2 units.
       const float mt = xor32_max(max16(x));
       const bool fresh = m_ref == -INFINITY;
       const bool need = fresh || xor32_max(ovf) > 0.f || mt > c_ref + kSnap;

@@ -184,7 +184,8 @@ __global__ __launch_bounds__(256) void transition_prep_kernel(TransitionArgs a) 
 // served by the 8 / R waves w / R, each passing every (8 / R)-th chunk.  Each
 // wave streams its chunks' planes through 16 KB of LDS of its own, four 4 KB
 // steps deep, with no barriers; the partial outputs are added through LDS in
-// wave order.  Bound by the planes from L2 (R 384 KB per CU and chunk).
+// wave order.  Bound by the planes from L2 (each wave reads 2 R chunks of 48 KB:
+// 768 R KB per tile).
 //
 // The rows that do not fill a round of full tiles take the smallest of these
 // that one more round covers: at N = 384 the last 64 of 576 tiles as 256
