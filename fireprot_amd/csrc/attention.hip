@@ -75,8 +75,8 @@
 // (B = 64, N = 1536: 786 us for a NaN in the first tile, 406 on the planes); a
 // value or range that only the last tiles or the sums show costs both, 1.2 ms.
 //
-// Bound: VALU issue beside the matrix cores (about 170 VALU instructions and
-// 12 MFMAs per wave and tile).  At B = 512, N = 1536: 3.13 ms; on the FP32
+// Bound: VALU issue beside the matrix cores (236 VALU instructions and 12 MFMAs
+// per wave and tile; VALU 86% busy, matrix cores 31%).  At B = 512, N = 1536: 3.13 ms; on the FP32
 // matrix cores, which never overlap with VALU work, 5.39 ms.  N = 384 176 us
 // against 304.
 #include "attn_common.hpp"

@@ -21,10 +21,12 @@
 // and split once, each row operand read from LDS serves both blocks, and
 // the two blocks are the two independent accumulation chains.
 //
-// Bound: MFMA issue plus VALU (48 MFMAs and about 450 VALU instructions per
-// wave and tile, which overlap only in part).  With a work-group per slice,
-// both normalising the tile, and its rows dealt over half as many streams:
-// 700 us at N = 1000, 48 at N = 256, 45 at N = 160; now 540, 43, 30.
+// Bound: MFMA issue plus VALU (48 MFMAs and 350 VALU instructions per wave and
+// tile; at N = 1000 busy 44% and 51% of the time, a third of the former
+// together), at small N the weights' way in and waits.  With a work-group per
+// slice, both normalising the tile, and its rows dealt over half as many
+// streams: 700 us at N = 1000, 48 at N = 256, 45 at N = 160; now 490 to 580 by
+// box, 43, 30.
 //
 // The pipeline is that of projection_block_kernel: LayerNorm 16
 // lanes per row, raw rows staged through LDS so that a row load is waited

@@ -160,11 +160,11 @@ typedef __bf16 XPlane[kRows][kPlaneRow];
 // accumulation chains.  The LayerNorm affine and the triangle-bias weights
 // are read from LDS tile by tile.
 //
-// Bound: MFMA issue, VALU and the stores of 2 KB per row (q, k, v and g, 512
-// bytes each, and 32 of bias), which overlap only in part at two waves per
-// SIMD.  As two work-groups per tile, 256 columns and one LayerNorm each, over
+// Bound: the stores of 2 KB per row (q, k, v and g, 512 bytes each, and 32 of
+// bias; at N = 1536 6.2 GB of traffic at 3.8 TB/s), MFMA issue and VALU (27%
+// and 32% busy), which overlap only in part at two waves per SIMD.  As two work-groups per tile, 256 columns and one LayerNorm each, over
 // the padded key tiles too, the launch took 1844 us at N = 1536, 250 at N =
-// 512, 64 at N = 256 and 44 at N = 160; now 1680, 222, 52 and 32.
+// 512, 64 at N = 256 and 44 at N = 160; now 1630 to 1700, 222, 52 and 32.
 constexpr int kBlockWaves = 8;
 __global__ __launch_bounds__(kBlockWaves * 64, 1) void projection_block_kernel(ProjArgs a,
                                                                                int tiles_j,
