@@ -782,10 +782,11 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
         const int c = 8 * rr + 4 * half;  // channels c..c+3 of head h
-        f32x4 ov = {__builtin_ldexpf(o[4 * rr + 0], -ev) / l_tot,
-                    __builtin_ldexpf(o[4 * rr + 1], -ev) / l_tot,
-                    __builtin_ldexpf(o[4 * rr + 2], -ev) / l_tot,
-                    __builtin_ldexpf(o[4 * rr + 3], -ev) / l_tot};
+        // the mean first: the sum itself may pass the largest float once unscaled
+        f32x4 ov = {__builtin_ldexpf(o[4 * rr + 0] / l_tot, -ev),
+                    __builtin_ldexpf(o[4 * rr + 1] / l_tot, -ev),
+                    __builtin_ldexpf(o[4 * rr + 2] / l_tot, -ev),
+                    __builtin_ldexpf(o[4 * rr + 3] / l_tot, -ev)};
         *(f32x4*)(a.out + (((int64_t)b * a.n + jq) * kHeads + h) * kHeadDim + c) = ov;
       }
     }

@@ -128,3 +128,17 @@ def test_non_finite_inputs_cost_no_more_than_fp32_products():
     broken = min(seconds() for _ in range(3))
     print(f"finite {finite:.3f} ms, non-finite {broken:.3f} ms", flush=True)
     assert broken <= 3.0 * finite, (broken, finite)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_values_near_the_largest_float(masked):
+    """A weighted mean of representable values is representable: nothing on the
+    way to it (the sum before its division) may overflow."""
+    n = 100
+    q, k, v, bias = _inputs(2, n, 19)
+    v *= 3e38 / v.abs().max()
+    mask = torch.full((2, n), -3.0, device="cuda") if masked else None
+    out = _run(q, k, v, bias, mask)
+    assert torch.isfinite(out).all()
+    ref = _torch(q, k, v, bias, mask, torch.float64)
+    assert ((out.double() - ref).abs().max() / ref.abs().max()).item() <= 2e-6
