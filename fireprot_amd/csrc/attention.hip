@@ -38,9 +38,10 @@
 // natural units, the native order (patches/protenix/0005-*.patch:36-45;
 // kernels/amd/fireprot_softmax_fp32.cpp:33-35).  These logits are quantised to
 // the FP32 spacing of -1e9 (64), and this order reproduces which keys tie at
-// the max.  Weights are exp2(fma(x, log2 e, -c)) with c = fl(m log2 e) of a
-// lazy running max m (rescaled when a tile max exceeds it by 2^8), so equal
-// logits get equal weights.
+// the max.  Weights are exp2(fma(x, log2 e, -c) - s) with c = fl(m log2 e) of a
+// lazy running max m (rescaled when a tile max exceeds it by 2^8) and s = m
+// log2(e) - c, so equal logits get equal weights, and the largest is in range
+// however far c is rounded (by up to 2^11 at 3e10).
 //
 // A row whose logits are all -inf gives NaN, as torch.softmax does.  fp16
 // planes cannot carry an infinity beside finite values (its residual is NaN),
@@ -190,6 +191,7 @@ __device__ __forceinline__ void attend_f32(const AttnArgs& a, int b, int h, int 
     constexpr bool kExact = decltype(exact_tag)::value;
     float m_ref = -INFINITY;  // largest tile max when the reference was last looked at
     float c_ref = 0.f;        // the reference, in log2 units
+    float s_ref = 0.f;        // exact path: m_ref log2(e) - c_ref, what c_ref's rounding left
     bool has_ref = false;     // uniform per wave, as big
     bool big = false;
     // As in the planes' path, fast rows round logits past 2^22 (big) to log2
@@ -219,11 +221,14 @@ __device__ __forceinline__ void attend_f32(const AttnArgs& a, int b, int h, int 
         if (__any(mt > m_ref + kRescaleNat)) {
           const float m_new = __builtin_elementwise_maximum(m_ref, mt);
           const float c_new = m_new == -INFINITY ? 0.f : m_new * kLog2e;
-          rescale(m_ref == -INFINITY ? 0.f : exp2_fast(c_ref - c_new));
+          rescale(m_ref == -INFINITY ? 0.f : exp2_fast((m_ref - m_new) * kLog2e));
           m_ref = m_new;
           c_ref = c_new;
+          s_ref = m_new == -INFINITY ? 0.f : __builtin_fmaf(m_new, kLog2e, -c_new);
         }
-        weights(x);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          x[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref) - s_ref);
         l_run += sum16(x);
         return;
       }
@@ -606,7 +611,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       // when the reference was last looked at (-inf: none yet).
       float m_ref = -INFINITY;
       float c_ref = 0.f;
-      float w_ref = 1.f;     // exact path: 2^-(m_ref log2(e) - c_ref)
+      float s_ref = -kShift; // exact path: m_ref log2(e) - c_ref, what c_ref's rounding left, - kShift
       bool has_ref = false;  // uniform per wave, as big
       bool big = false;
       // Logits x in natural units -> the weights' planes.
@@ -623,12 +628,12 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
             l_run *= alpha;
             m_ref = m_new;
             c_ref = c_new;
-            w_ref = m_new == -INFINITY ? 1.f : exp2_fast(-__builtin_fmaf(m_new, kLog2e, -c_new));
+            s_ref = (m_new == -INFINITY ? 0.f : __builtin_fmaf(m_new, kLog2e, -c_new)) - kShift;
           }
-          // P = p w_ref is at most 2^8; the planes hold P 2^kShift, the sum P 2^kShift too
-          const float f = w_ref * 128.0f;
+          // The weights are at most 2^8; the planes and the sum hold them times 2^kShift.
 #pragma unroll
-          for (int r = 0; r < 16; ++r) p[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref)) * f;
+          for (int r = 0; r < 16; ++r)
+            p[r] = exp2_fast(__builtin_fmaf(x[r], kLog2e, -c_ref) - s_ref);
           l_run += sum16(p);
         } else {
           // Logits past 2^22 (big) are rounded to log2 units before the

@@ -142,3 +142,29 @@ def test_values_near_the_largest_float(masked):
     assert torch.isfinite(out).all()
     ref = _torch(q, k, v, bias, mask, torch.float64)
     assert ((out.double() - ref).abs().max() / ref.abs().max()).item() <= 2e-6
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("gain", [1.0, 1e6, 3e10, 1e30])
+def test_rows_without_an_unmasked_key_at_any_logit_size(gain, wide):
+    """The logits of a fully masked row keep their distances at any size: from
+    3e10 on, log2(e) times the largest is rounded by more than an exponential
+    can hold.  wide: on the FP32 matrix cores too."""
+    n = 100
+    q, k, v, bias = _inputs(2, n, 20)
+    bias = bias * gain
+    if wide:
+        v[:, 70] *= 1e9
+        bias[:, :, 70] -= 1e4 * gain
+    mask = torch.full((2, n), -1e9, device="cuda")
+    out = _run(q, k, v, bias, mask).double()
+    # the native order in float32, the rest in float64
+    s = torch.matmul(*(t.permute(0, 2, 1, 3).contiguous() if i == 0 else
+                       t.permute(0, 2, 3, 1).contiguous() for i, t in enumerate((q, k))))
+    x = ((s + mask[:, None, None, :]) + bias).double()
+    ref = torch.matmul(torch.softmax(x, -1), v.double().permute(0, 2, 1, 3).contiguous())
+    err = (out - ref.permute(0, 2, 1, 3)).abs().amax((1, 2, 3))
+    # q k flips a logit of the grid of 64 only where it lies near a midpoint: the sum
+    # with -1e9 rounds it away, and both sides add the same bias to the same number
+    assert torch.isfinite(out).all()
+    assert (err <= 2e-6 * ref.abs().amax((1, 2, 3))).all(), err
