@@ -71,8 +71,9 @@
 // Tiles of V further apart than 2^20 (kMaxSpread; padded keys holding anything
 // are the usual cause) go to FP32 as they are met.  So the planes' error is
 // relative to the largest output of the row and to the largest V of the
-// channel.  The looks cost 1.6% at N = 1536 (3080 to 3129 us) and at most
-// 0.6 us of 13 at N = 128.  attend_f32 runs at the rate of a kernel of its own
+// channel.  The looks cost 1.6% at N = 1536 (3080 to 3129 us; 3 to 4% with a
+// mask: B = 64 508 to 525 us where every key is masked) and at most 0.6 us of 13
+// at N = 128.  attend_f32 runs at the rate of a kernel of its own
 // (B = 64, N = 1536: 786 us for a NaN in the first tile, 406 on the planes); a
 // value or range that only the last tiles or the sums show costs both, 1.2 ms.
 //
