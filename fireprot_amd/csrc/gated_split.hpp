@@ -25,8 +25,8 @@
 // tile; at N = 1000 busy 44% and 51% of the time, a third of the former
 // together), at small N the weights' way in and waits.  With a work-group per
 // slice, both normalising the tile, and its rows dealt over half as many
-// streams: 700 us at N = 1000, 48 at N = 256, 45 at N = 160; now 490 to 580 by
-// box, 43, 30.
+// streams: 700 us at N = 1000, 48 at N = 256, 45 at N = 160; now 490 to 580
+// from card to card, 43, 30.
 //
 // The pipeline is that of projection_block_kernel: LayerNorm 16
 // lanes per row, raw rows staged through LDS so that a row load is waited

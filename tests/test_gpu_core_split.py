@@ -62,8 +62,9 @@ def test_tile_edges(n, masked):
 @pytest.mark.parametrize("scales", [(1e-6, 1.0, 1e4), (1e4, 1.0, 1e-6), (0.0, 1.0, 0.0),
                                     (1e-30, 1e-33, 1e-36)])
 def test_tiles_of_different_magnitudes(which, scales):
-    """Each 32-key tile at its own scale: V's exponent falls (O is rescaled)
-    and rises, a zero tile sets none, values far below the others stay."""
+    """Each 32-row block, the unit of an exponent, at its own scale: V's exponent
+    falls (O is rescaled) and rises, a zero tile sets none.  Scales that change
+    inside a block are test_gpu_core_range.py's."""
     n = 160
     q, k, v, bias = _inputs(2, n, 5)
     s = torch.tensor(scales, device="cuda")[(torch.arange(n, device="cuda") // 32) % 3]
