@@ -65,9 +65,12 @@
 //     weights, uniformly distributed errors of random sign).  A query whose
 //     largest |O'| over the channels is not 2^22 times that sum (kRowShare,
 //     kWeightShare) gets its weight from keys of V far below the largest (a
-//     masked key's, say): FP32.  Likewise when some channel's largest |V| is
-//     nonzero and below 1, 2^-14 or less of all: its error would pass 2^-25
-//     of it.
+//     masked key's, say): FP32.  (Equal weights round alike and their errors
+//     add up, N / sqrt(N / 3) times as much; so do the roundings of an FP32
+//     sum of N like terms, and the latter are the larger wherever |O'| passes
+//     2^14, as it does here from N = 192 on.)  Likewise FP32 when some
+//     channel's largest |V| is nonzero and below 1, 2^-14 or less of all: its
+//     error would pass 2^-25 of it.
 // Tiles of V further apart than 2^20 (kMaxSpread; padded keys holding anything
 // are the usual cause) go to FP32 as they are met.  So the planes' error is
 // relative to the largest output of the row and to the largest V of the
@@ -97,14 +100,17 @@ constexpr int kPlaneBytes = 2048;              // 32 rows of 64 bytes
 constexpr int kTileBytes = 4 * kPlaneBytes;    // K hi, K lo, V^T hi, V^T lo
 constexpr int kBiasBytes = 32 * kBk * 4;       // a wave's bias fragment
 constexpr float kPlaneMax = 32768.0f;          // bound on a lane's 16 scaled weights
-constexpr float kShift = 7.0f;                 // weights enter P.V as up to 2^7 and more
+// Weights enter P.V as up to 2^7 and more.  2^10 would resolve small ones eight times finer and
+// keep more rows off attend_f32, but moves the reference more often: 2 to 4% at logits of 4
+// standard deviations.
+constexpr float kShift = 7.0f;
 constexpr int64_t kMaxBiasStride = 1 << 25;    // 31 rows within 32-bit byte offsets
 constexpr float kBigLogit = 4194304.0f;        // 2^22: past it, references take no shift
-// Range of the planes (file comment); 2^22 times 2^-25 and 2^-25 2^14 / sqrt(3).
+// Range of the planes (file comment).
 constexpr float kMaxProduct = 1024.0f;
 constexpr float kEvenShare = 0x1p-8f;
-constexpr float kRowShare = 0.125f;
-constexpr float kWeightShare = 1182.4f;
+constexpr float kRowShare = 0.125f;      // 2^22 2^-25
+constexpr float kWeightShare = 1182.4f;  // 2^22 2^-25 2^14 / sqrt(3)
 constexpr int kMaxSpread = 20;
 constexpr int kNoExp = 141;  // V's exponent while every tile was zero
 
@@ -612,7 +618,7 @@ __global__ __launch_bounds__(kThreads, 4) void attention_kernel(AttnArgs a, int 
       // when the reference was last looked at (-inf: none yet).
       float m_ref = -INFINITY;
       float c_ref = 0.f;
-      float s_ref = -kShift; // exact path: m_ref log2(e) - c_ref, what c_ref's rounding left, - kShift
+      float s_ref = -kShift;  // exact path: m_ref log2(e) - c_ref, what its rounding left, - shift
       bool has_ref = false;  // uniform per wave, as big
       bool big = false;
       // Logits x in natural units -> the weights' planes.

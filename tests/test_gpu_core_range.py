@@ -126,3 +126,25 @@ def test_logit_scales(gain):
     err, base = (out - ref).abs().max().item(), (low - ref).abs().max().item()
     print(f"gain {gain}: err {err:.3e}, FP32 torch {base:.3e}", flush=True)
     assert err <= max(2e-6 * ref.abs().max().item(), 2.0 * base), (err, base)
+
+
+@pytest.mark.parametrize("ratio", [16.0, 60.0, 250.0, 4000.0])
+@pytest.mark.parametrize("n", [260, 1536])
+def test_many_equal_small_weights_on_large_values(n, ratio):
+    """One key takes nearly all weight, the others share one tiny weight on
+    values `ratio` times its own: equal terms round alike, so errors add up
+    instead of averaging out, n times half an ulp in an FP32 sum of n terms
+    (the bar's 2^-24: a sum between the powers of two)."""
+    q, k, v, bias = _inputs(1, n, 29)
+    q.zero_()
+    v.fill_(ratio)
+    v[:, 7] = 1.0
+    bias.zero_()
+    for i, drop in enumerate((14.0, 16.5, 18.3, 19.7)):  # weights of 2^-20 to 2^-28
+        bias[i] = -drop
+    bias[:, :, 7] = 0.0
+    out = _run(q, k, v, bias).double()
+    ref = _torch(q, k, v, bias, None, torch.float64)
+    worst = ((out - ref).abs() / ref.abs()).max().item()
+    print(f"n {n} ratio {ratio}: {worst:.2e}", flush=True)
+    assert worst <= n * 2.0 ** -24, worst
