@@ -106,9 +106,9 @@ def test_bias_rows_beyond_32_bit_offsets():
 
 
 def test_non_finite_inputs_cost_no_more_than_fp32_products():
-    """A batch whose every row holds a NaN runs on the FP32 matrix cores (1.8
-    times the planes' time at N = 1536), not key by key (over 20 times).  Three
-    times the finite time leaves room for noise."""
+    """A batch whose every row holds a NaN runs on the FP32 matrix cores (2.2
+    times the finite time here), not key by key (19 times).  Five times leaves
+    room for noise on either side."""
     q, k, v, bias = _inputs(64, 512, 17)
 
     def seconds():
@@ -128,7 +128,7 @@ def test_non_finite_inputs_cost_no_more_than_fp32_products():
     v[:, 300, 0::3, 5] = float("nan")
     broken = min(seconds() for _ in range(3))
     print(f"finite {finite:.3f} ms, non-finite {broken:.3f} ms", flush=True)
-    assert broken <= 3.0 * finite, (broken, finite)
+    assert broken <= 5.0 * finite, (broken, finite)
 
 
 @pytest.mark.parametrize("masked", [False, True])
